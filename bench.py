@@ -116,8 +116,7 @@ def copy_calibration(nbytes):
     print(json.dumps({"copy_bytes": nbytes, "copies": 5}), flush=True)
 
 
-STAGING = {0: "registers -> padded LDS, 8x4x4 parts", 1: "direct global -> LDS, 8x4x4 parts",
-           2: "direct global -> LDS, 8x4x8 parts"}
+STAGING = {0: "16x4x2 or 16x4x4 parts by launch size", 1: "16x4x2 parts", 2: "16x4x4 parts"}
 
 
 def level_tuning(ga, lvl, times=None):

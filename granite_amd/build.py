@@ -34,7 +34,7 @@ FLAGS = [
 
 def build(verbose: bool = False, out: str = LIB, defines=()) -> str:
     """Compile every source into `out` (default: the in-tree library); always recompiles.
-    `defines` are extra -D macros (tile shape and prefetch depth of the stage kernel)."""
+    `defines` are extra -D macros (tile shape of the stage kernels)."""
     tmp = out + ".tmp"
     cmd = [HIPCC, *FLAGS, *["-D" + d for d in defines], "-I", os.path.join(ROOT, "include"), *SOURCES, "-o", tmp]
     if verbose:

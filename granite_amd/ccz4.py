@@ -22,7 +22,7 @@ PREC_FP64, PREC_MIXED = 0, 1
 # tuned choices (enum gr_tune_kind)
 TUNE_STAGE, TUNE_GHOST, TUNE_TRANSFER = 0, 1, 2
 GROUP_CHOICES = (1, 2, 4, 11)
-STAGE_VARIANTS = 3  # FP64 staging: 0 registers, 1 direct LDS (8x4x4 parts), 2 direct LDS (8x4x8 parts)
+STAGE_VARIANTS = 3  # FP64 parts: 0 by launch size, 1 always 16x4x2, 2 always 16x4x4
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 
@@ -491,7 +491,7 @@ class Level:
         self._e.check(self._e.lib.gr_level_set_mixed_policy(self._h, float(chi_fp64_below)))
 
     def autotune(self, params: CCZ4Params, dt):
-        """Time the stage-kernel staging variants (per group of equal spacing) and the ghost
+        """Time the stage kernel's part shapes (per group of equal spacing) and the ghost
         fill's field groups on this level, keep the fastest (gr_level_autotune). Returns
         {"stage": [[ms per variant, None where not applicable] per group], "ghost": {groups: ms}}."""
         cap = 256

@@ -377,7 +377,7 @@ int gr_ccz4_constraints(gr_engine* e, const gr_geom* geom, const double* u, doub
 
 // ---------------------------------------------------------------------------------------
 // Tuning table: the kernel variant chosen for each (choice, block-size class, precision).
-// Choices: the FP64 stage kernel's staging variant (0 registers, 1 direct LDS), the ghost
+// Choices: the FP64 stage kernel's parts (0 by launch size, 1 small, 2 large), the ghost
 // fill's field groups (1, 2, 4, 11) and the AMR transfers' field groups (1, 2, 4, 11). The
 // class is the mean interior cells per block: < 24^3, < 48^3, < 96^3, larger. Levels and
 // hierarchies read the table when they are created; gr_level_autotune / gr_hierarchy_autotune
@@ -525,10 +525,8 @@ int gr_level_create(gr_engine* e, int nblocks, const gr_geom* geoms, gr_level** 
         if (st != hipSuccess) break;
         st = build_batch(L, G.blocks, G.table, &G.d_table, &G.d_tile_block, &G.d_ghost_wg_block, &G.batch);
         if (st == hipSuccess) st = hipMalloc((void**)&G.flags, G.batch.ntiles);
-        // without a table entry: the direct-to-LDS staging in 8x4x8 parts where the rows allow
-        // it and the launch is large enough to fill the machine (at least 40^3 cells), else
-        // the register staging (below that a stage launch is latency-bound: measured 10% faster
-        // in variant 0 for single blocks up to 32^3, 22% slower from 48^3)
+        // without a table entry: the large parts where the rows allow forcing them and the launch is
+        // large enough to fill the machine (at least 40^3 cells), else the launch's own choice
         double cells = 0.0;
         for (int i : G.blocks) cells += (double)L->blk[i].n[0] * L->blk[i].n[1] * L->blk[i].n[2];
         int v = (G.batch.pairs_ok && cells >= 40.0 * 40 * 40) ? 2 : 0;
@@ -946,7 +944,7 @@ int gr_level_rhs(gr_level* L, int b, const gr_ccz4_params* prm, int precision, d
         for (int i : G.blocks)
             if (i == b) {
                 flags = G.flags;
-                B.variant = G.batch.variant; // the staging variant of the block's group
+                B.variant = G.batch.variant; // the stage form of the block's group
             }
     GR_HIP(e, stage_batch(L, B, flags, sel, prm, gr::MODE_RHS, gr::StageCoef{0.0, 0.0, 0.0}, precision));
     GR_HIP(e, hipMemcpyAsync(host_rhs, L->s1[b], n * sizeof(double), hipMemcpyDeviceToHost, e->stream));
@@ -1254,9 +1252,9 @@ int gr_level_set_tuning(gr_level* L, int kind, int group, int value) {
     gr_engine* e = L->eng;
     if (kind == GR_TUNE_STAGE) {
         if (group < 0 || group >= (int)L->groups.size()) return fail(e, GR_ERR_ARG, "group index out of range");
-        if (!tune_valid(kind, value)) return fail(e, GR_ERR_ARG, "unknown staging variant");
+        if (!tune_valid(kind, value)) return fail(e, GR_ERR_ARG, "unknown stage form");
         if (value != 0 && !L->groups[group].batch.pairs_ok)
-            return fail(e, GR_ERR_ARG, "direct LDS staging needs even row lengths and 16-byte aligned buffers");
+            return fail(e, GR_ERR_ARG, "a fixed part shape needs even row lengths and 16-byte aligned buffers");
         L->groups[group].batch.variant = value;
     } else if (kind == GR_TUNE_GHOST) {
         if (!tune_valid(kind, value)) return fail(e, GR_ERR_ARG, "ghost field groups must be 1, 2, 4 or 11");

@@ -77,14 +77,22 @@ struct Stencil {
 };
 
 // Index strides of a staged array along x, y, z. The LDS tile uses compile-time strides
-// so that every stencil tap is an immediate offset from one base address.
+// so that every stencil tap is an immediate offset from one base address. READS_FIRST asks the
+// compiler to issue a field's reads ahead of its arithmetic (eval_field).
 template <int SX, int SY, int SZ>
 struct FixedStrides {
+    static constexpr bool READS_FIRST = false;
     __host__ __device__ static constexpr long q(int d) { return d == 0 ? SX : (d == 1 ? SY : SZ); }
+    // value k cells off along axis d
+    template <typename R>
+    __host__ __device__ static R at(const R* s, int d, int k) { return s[k * q(d)]; }
 };
 struct RuntimeStrides {
+    static constexpr bool READS_FIRST = false;
     long s[3];
     __host__ __device__ long q(int d) const { return s[d]; }
+    template <typename R>
+    __host__ __device__ R at(const R* p, int d, int k) const { return p[k * s[d]]; }
 };
 
 struct CellParams {
@@ -123,11 +131,11 @@ __host__ __device__ GR_INLINE void pin(R& x) {
 // free of FMA contraction, so fields whose RHS is dominated by dissipation (a constant or
 // noisy metric) reproduce the reference to the last bit.
 template <typename R>
-__host__ __device__ GR_INLINE R ko_axis_ordered(R acc, const R* kw, R m3, R m2, R m1, R c, R p1, R p2, R p3) {
+__host__ __device__ GR_INLINE R ko_axis_ordered(bool first, R acc, const R* kw, R m3, R m2, R m1, R c, R p1, R p2, R p3) {
 #ifdef __clang__
 #pragma clang fp contract(off)
 #endif
-    acc = acc + kw[0] * m3;
+    acc = first ? kw[0] * m3 : acc + kw[0] * m3;
     acc = acc + kw[1] * m2;
     acc = acc + kw[2] * m1;
     acc = acc + kw[3] * c;
@@ -137,34 +145,82 @@ __host__ __device__ GR_INLINE R ko_axis_ordered(R acc, const R* kw, R m3, R m2, 
     return acc;
 }
 
+// Advection sum of one cell: sum over axes of beta^d times the blend w * upwind + (1 - w) *
+// centred derivative, with the factors that no field changes taken out of it: up[d] = -w |beta^d| /
+// (12 h_d) for the upwind polynomial (the forward one's sign is beta's, the backward one is
+// negated) and cen[d] = (1 - w) beta^d for the centred derivative. side() picks the tap on the
+// upwind side: on the GPU by a lane mask and a conditional move, which the compiler would
+// otherwise turn into a branch per axis and field that splits the field's code into pieces
+// it schedules one by one.
+template <typename R>
+struct Advection {
+    static constexpr bool FOLDED = sizeof(R) == 8; // the FP32 form keeps beta and w apart (below)
+    R up[3], cen[3];
+    R be[3], w;
+    bool neg[3]; // beta^d >= 0: the backward side (per lane; also false for NaN)
+#ifdef __HIP_DEVICE_COMPILE__
+    unsigned long long back[3]; // the same as a lane mask
+    __device__ __forceinline__ static unsigned move(unsigned long long m, unsigned b, unsigned f) {
+        unsigned r;
+        asm("v_cndmask_b32 %0, %1, %2, %3" : "=v"(r) : "v"(f), "v"(b), "s"(m));
+        return r;
+    }
+    // the FP32 form's code is scheduled better with the compiler's own selects and the blend at the
+    // end (measured on a 128^3 stage: 505 us against 580)
+    __device__ __forceinline__ float side(int d, float b, float f) const { return neg[d] ? b : f; }
+    __device__ __forceinline__ double side(int d, double b, double f) const {
+        const unsigned lo = move(back[d], (unsigned)__double2loint(b), (unsigned)__double2loint(f));
+        const unsigned hi = move(back[d], (unsigned)__double2hiint(b), (unsigned)__double2hiint(f));
+        return __hiloint2double((int)hi, (int)lo);
+    }
+#else
+    __host__ __device__ R side(int d, R b, R f) const { return neg[d] ? b : f; }
+#endif
+    __host__ __device__ GR_INLINE void set(const R beta[3], R blend, const R ih[3]) {
+        w = blend;
+        for (int d = 0; d < 3; ++d) {
+            be[d] = beta[d];
+            neg[d] = beta[d] >= R(0);
+#ifdef __HIP_DEVICE_COMPILE__
+            back[d] = __builtin_amdgcn_ballot_w64(neg[d]);
+#endif
+            up[d] = w * ((neg[d] ? -ih[d] : ih[d]) * beta[d]);
+            cen[d] = (R(1) - w) * beta[d];
+        }
+    }
+};
+
 // All stencils of one field at one cell: 4th-order centred first derivative, one-sided
 // 5-point upwind derivative picked by the sign of beta (used only through the advection
 // sum), 7-point Kreiss-Oliger sum, and (D2) the 4th-order pure and 2nd-order mixed second
 // derivatives. dd is stored by symmetric pair index. KO_EXACT selects the reference's
 // accumulation order for the dissipation sum; otherwise it is grouped by symmetric taps.
 template <bool D2, bool KO_EXACT, typename R, class ST>
-__host__ __device__ GR_INLINE void eval_field(const R* s, const Stencil<R>& K, const ST& st, const R be[3], R w,
+__host__ __device__ GR_INLINE void eval_field(const R* s, const Stencil<R>& K, const ST& st, const Advection<R>& B,
                                               R d1[3], R dd[6], R& adv, R& ko) {
     const R c = s[0];
     R upS = R(0), cenS = R(0);
-    ko = R(0);
+    adv = R(0);
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
-        const long q = st.q(d);
-        const R m1 = s[-q], p1 = s[q], m2 = s[-2 * q], p2 = s[2 * q];
-        const R m3 = s[-3 * q], p3 = s[3 * q], m4 = s[-4 * q], p4 = s[4 * q];
+        const R m1 = st.at(s, d, -1), p1 = st.at(s, d, 1), m2 = st.at(s, d, -2), p2 = st.at(s, d, 2);
+        const R m3 = st.at(s, d, -3), p3 = st.at(s, d, 3), m4 = st.at(s, d, -4), p4 = st.at(s, d, 4);
         const R dv = K.ih[d] * (-p2 + R(8) * p1 - R(8) * m1 + m2);
         d1[d] = dv;
         // backward stencil for beta >= 0 equals the forward one mirrored and negated
-        const bool bw = be[d] >= R(0);
-        const R g1 = bw ? m1 : p1, g2 = bw ? m2 : p2, g3 = bw ? m3 : p3, g4 = bw ? m4 : p4;
-        const R up = (bw ? -K.ih[d] : K.ih[d]) * (R(-25) * c + R(48) * g1 - R(36) * g2 + R(16) * g3 - R(3) * g4);
-        upS += be[d] * up;
-        cenS += be[d] * dv;
+        const R g1 = B.side(d, m1, p1), g2 = B.side(d, m2, p2), g3 = B.side(d, m3, p3), g4 = B.side(d, m4, p4);
+        const R poly = R(-25) * c + R(48) * g1 - R(36) * g2 + R(16) * g3 - R(3) * g4;
+        if (B.FOLDED) {
+            adv += B.up[d] * poly;
+            adv += B.cen[d] * dv;
+        } else {
+            upS += B.be[d] * ((B.neg[d] ? -K.ih[d] : K.ih[d]) * poly);
+            cenS += B.be[d] * dv;
+        }
         if (KO_EXACT)
-            ko = ko_axis_ordered(ko, K.kw[d], m3, m2, m1, c, p1, p2, p3);
+            ko = ko_axis_ordered(d == 0, ko, K.kw[d], m3, m2, m1, c, p1, p2, p3);
         else
-            ko += K.ko[d] * ((m3 + p3) - R(6) * (m2 + p2) + R(15) * (m1 + p1) - R(20) * c);
+            ko = (d == 0 ? R(0) : ko) + K.ko[d] * ((m3 + p3) - R(6) * (m2 + p2) + R(15) * (m1 + p1) - R(20) * c);
         if (D2) dd[sym(d, d)] = K.ih2[d] * (-p2 + R(16) * p1 - R(30) * c + R(16) * m1 - m2);
     }
     if (D2) {
@@ -173,13 +229,12 @@ __host__ __device__ GR_INLINE void eval_field(const R* s, const Stencil<R>& K, c
         dd[2] = K.ihh[1] * (s[x + z] - s[x - z] - s[-x + z] + s[-x - z]);
         dd[4] = K.ihh[2] * (s[y + z] - s[y - z] - s[-y + z] + s[-y - z]);
     }
-    adv = w * upS + (R(1) - w) * cenS;
+    if (!B.FOLDED) adv = B.w * upS + (R(1) - B.w) * cenS;
 #ifdef __HIP_DEVICE_COMPILE__
-    // scheduling hint for the field's code: its LDS reads go out before its arithmetic, so the
-    // reads wait in two batches instead of four and the second batch's latency is covered by
-    // the first batch's arithmetic (results unchanged: the same instructions, reordered)
-    __builtin_amdgcn_sched_group_barrier(0x100, 40, 0); // LDS reads
-    __builtin_amdgcn_sched_group_barrier(0x002, 400, 0); // then VALU
+    if constexpr (ST::READS_FIRST) {
+        __builtin_amdgcn_sched_group_barrier(0x100, 40, 0); // LDS reads
+        __builtin_amdgcn_sched_group_barrier(0x002, 400, 0); // then VALU
+    }
 #endif
     pin(adv);
     pin(ko);
@@ -233,7 +288,8 @@ __host__ __device__ GR_INLINE void ccz4_cell(Stager& S, Sink& O, const Stencil<R
         gu[4] = R((g[1] * g[2] - g[0] * g[4]) * idet);
         gu[5] = R((g[0] * g[3] - g[1] * g[1]) * idet);
     }
-    const R w = R(0.5) * (R(1) + tanh_((chi - R(P.chi_c)) / R(P.chi_w)));
+    Advection<R> B;
+    B.set(be, R(0.5) * (R(1) + tanh_((chi - R(P.chi_c)) / R(P.chi_w))), K.ih);
 
     R d1[3], dd[6], adv, ko;
 
@@ -247,7 +303,7 @@ __host__ __device__ GR_INLINE void ccz4_cell(Stager& S, Sink& O, const Stencil<R
     R dbe[3][3], ddiv[3] = {R(0), R(0), R(0)};
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
-        eval_field<true, KO_EXACT>(S.field(BX + c), K, S.strides(), be, w, d1, dd, adv, ko);
+        eval_field<true, KO_EXACT>(S.field(BX + c), K, S.strides(), B, d1, dd, adv, ko);
         R t5 = R(0);
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
@@ -273,7 +329,7 @@ __host__ __device__ GR_INLINE void ccz4_cell(Stager& S, Sink& O, const Stencil<R
 #pragma unroll
     for (int p = 0; p < 6; ++p) {
         const int a = sym_a(p), b = sym_b(p);
-        eval_field<true, KO_EXACT>(S.field(GXX + p), K, S.strides(), be, w, dgt[p], dd, adv, ko);
+        eval_field<true, KO_EXACT>(S.field(GXX + p), K, S.strides(), B, dgt[p], dd, adv, ko);
         R r1 = R(0);
 #pragma unroll
         for (int q = 0; q < 6; ++q) r1 += ((q == 0 || q == 3 || q == 5) ? R(-0.5) : R(-1)) * gu[q] * dd[q];
@@ -322,7 +378,7 @@ __host__ __device__ GR_INLINE void ccz4_cell(Stager& S, Sink& O, const Stencil<R
     R dchi[3];
     {
         R ddchi[6];
-        eval_field<true, KO_EXACT>(S.field(CHI), K, S.strides(), be, w, dchi, ddchi, adv, ko);
+        eval_field<true, KO_EXACT>(S.field(CHI), K, S.strides(), B, dchi, ddchi, adv, ko);
         O.put(CHI, (R(2) / R(3)) * chi * (alpha * Ktr - divb) + adv, ko, chi_raw);
         R lapchi = R(0), gradchi2 = R(0);
 #pragma unroll
@@ -348,7 +404,7 @@ __host__ __device__ GR_INLINE void ccz4_cell(Stager& S, Sink& O, const Stencil<R
     R dal[3], DDa[6];
     {
         R ddal[6];
-        eval_field<true, KO_EXACT>(S.field(ALPHA), K, S.strides(), be, w, dal, ddal, adv, ko);
+        eval_field<true, KO_EXACT>(S.field(ALPHA), K, S.strides(), B, dal, ddal, adv, ko);
         O.put(ALPHA, R(-2) * alpha * Ktr + adv, ko, alpha);
 #pragma unroll
         for (int p = 0; p < 6; ++p) {
@@ -434,7 +490,7 @@ __host__ __device__ GR_INLINE void ccz4_cell(Stager& S, Sink& O, const Stencil<R
     // ---- K (ccz4.cpp:621-652); its gradient completes T2 of Gamma-hat
     {
         R dK[3];
-        eval_field<false, KO_EXACT>(S.field(KTR), K, S.strides(), be, w, dK, dd, adv, ko);
+        eval_field<false, KO_EXACT>(S.field(KTR), K, S.strides(), B, dK, dd, adv, ko);
         const R matter = HAS_SRC ? R(4) * R(PI) * alpha * (R(src.rho) + R(src.S)) : R(0);
         O.put(KTR,
               -plap + alpha * (AA + Ktr * Ktr / R(3)) + matter + R(P.kappa1) * (R(1) - R(P.kappa2)) * alpha * Theta + adv,
@@ -455,7 +511,7 @@ __host__ __device__ GR_INLINE void ccz4_cell(Stager& S, Sink& O, const Stencil<R
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
         R advq, koq;
-        eval_field<false, KO_EXACT>(S.field(GHX + q), K, S.strides(), be, w, d1, dd, advq, koq);
+        eval_field<false, KO_EXACT>(S.field(GHX + q), K, S.strides(), B, d1, dd, advq, koq);
 #pragma unroll
         for (int p = 0; p < 6; ++p) {
             const int a = sym_a(p), b = sym_b(p);
@@ -478,7 +534,7 @@ __host__ __device__ GR_INLINE void ccz4_cell(Stager& S, Sink& O, const Stencil<R
     pin(Rs);
 
     // ---- Theta (ccz4.cpp:654-665)
-    eval_field<false, KO_EXACT>(S.field(THETA), K, S.strides(), be, w, d1, dd, adv, ko);
+    eval_field<false, KO_EXACT>(S.field(THETA), K, S.strides(), B, d1, dd, adv, ko);
     {
         const R rho = HAS_SRC ? R(src.rho) : R(0);
         O.put(THETA,
@@ -492,7 +548,7 @@ __host__ __device__ GR_INLINE void ccz4_cell(Stager& S, Sink& O, const Stencil<R
 #pragma unroll
     for (int p = 0; p < 6; ++p) {
         const int a = sym_a(p), b = sym_b(p);
-        eval_field<false, KO_EXACT>(S.field(AXX + p), K, S.strides(), be, w, d1, dd, adv, koA[p]);
+        eval_field<false, KO_EXACT>(S.field(AXX + p), K, S.strides(), B, d1, dd, adv, koA[p]);
         const R t1 = HAS_SRC ? chi * (XA[p] - alpha * R(8) * R(PI) * R(src.Sij[p])) : chi * XA[p];
         R Aub[3]; // A^q_b = g^qr A_rb
 #pragma unroll

@@ -1,21 +1,18 @@
-// gfx950 kernels of the CCZ4 RHS + SSP-RK3 stage engine (FP64 form).
+// gfx950 kernels of the CCZ4 RHS + SSP-RK3 stage engine.
 //
-// Stage kernel layout: one workgroup per tile of TX x TY x TZ interior cells, one thread
-// per cell. The 22 fields are streamed one at a time through an LDS box holding the tile
-// plus the stencil halo (4 cells along each axis, 1 cell on the edges used by the mixed
-// second derivatives); each field is read from HBM once per tile in coalesced rows along x.
-// The per-cell arithmetic is ccz4_cell.hpp; the RK3 combine, the floors and (last stage)
-// the algebraic constraints are applied to each value before it is stored, so one launch
-// per stage reads the stage input and u^n and writes the new stage state.
+// Stage kernel layout: one workgroup per part of a launch tile, one thread per cell. The 22
+// fields are streamed one at a time through an LDS box holding the part plus the stencil halo (4
+// cells along each axis, 1 cell on the edges used by the mixed second derivatives). The per-cell
+// arithmetic is ccz4_cell.hpp; the RK3 combine, the floors and (last stage) the algebraic
+// constraints are applied to each value before it is stored, so one launch per stage reads the
+// stage input and u^n and writes the new stage state.
 #include "kernels.hpp"
 
 #include <cstdint>
 
 // tile shape (overridable at build time): a tile of GR_TILE_X x Y x Z cells is the unit of
 // the launch bookkeeping and of the mixed-precision classification and kernel (one thread
-// per cell); the FP64 kernel, whose registers allow one wave per SIMD, runs each tile as
-// GR_FP64_SPLIT x GR_FP64_ZSPLIT workgroups of GR_TILE_X / GR_FP64_SPLIT x Y x
-// GR_TILE_Z / GR_FP64_ZSPLIT cells
+// per cell); the FP64 kernel runs each tile as parts (FP64_PARTS below)
 #ifndef GR_TILE_X
 #define GR_TILE_X 16
 #endif
@@ -25,20 +22,8 @@
 #ifndef GR_TILE_Z
 #define GR_TILE_Z 8
 #endif
-#ifndef GR_FP64_ZSPLIT
-#define GR_FP64_ZSPLIT 2
-#endif
-#ifndef GR_FP64_SPLIT
-#define GR_FP64_SPLIT 2
-#endif
-#ifndef GR_FP64_PREFETCH
-#define GR_FP64_PREFETCH 1
-#endif
 #ifndef GR_FP64_KO_EXACT
 #define GR_FP64_KO_EXACT 1
-#endif
-#ifndef GR_FP64_MIN_WAVES
-#define GR_FP64_MIN_WAVES 1
 #endif
 // parts of a tile along x the mixed kernel runs as separate workgroups (1 or 2)
 #ifndef GR_MIXED_SPLIT
@@ -46,21 +31,6 @@
 #endif
 #ifndef GR_MIXED_MIN_WAVES
 #define GR_MIXED_MIN_WAVES 1
-#endif
-#ifndef GR_LDS_PAD
-#define GR_LDS_PAD 1
-#endif
-// LDS layout of the FP64 parts: 0 = rows padded to a conflict-free pitch, lanes x-fastest
-// (55 KB for two buffers of an 8x4x4 part: two workgroups per CU); 1 = unpadded rows,
-// planes padded, lanes interleaved over y and z (38 KB: room for four workgroups per CU,
-// i.e. two waves per SIMD when the registers allow it)
-// field buffers of the direct-to-LDS staging, at most (2 or 3; fewer where more would not
-// leave two waves per SIMD room in the CU's LDS); the last stage's own limit
-#ifndef GR_DMA_BUFFERS
-#define GR_DMA_BUFFERS 3
-#endif
-#ifndef GR_DMA_BUFFERS_FINAL
-#define GR_DMA_BUFFERS_FINAL 2
 #endif
 #ifndef GR_MIXED_PREFETCH
 #define GR_MIXED_PREFETCH 1
@@ -93,16 +63,6 @@ __device__ __forceinline__ double gload(const gdouble* base, unsigned off) {
 __device__ __forceinline__ void gstore(gdouble* base, unsigned off, double v) {
     *(gdouble*)((gchar*)base + off) = v;
 }
-// the same load with the offset made opaque at the point of use, so that the 32-bit offset
-// reaches the load itself (scalar base + 32-bit vector offset, no 64-bit address add per
-// load) instead of a 64-bit copy of it hoisted out of the loop over fields
-__device__ __forceinline__ double gload_sv(const gdouble* base, unsigned off) {
-#ifdef __HIP_DEVICE_COMPILE__
-    asm volatile("" : "+v"(off));
-#endif
-    return *(const gdouble*)((const gchar*)base + off);
-}
-
 namespace {
 
 constexpr int HALO = 4;
@@ -154,7 +114,7 @@ __device__ __forceinline__ void algebraic_exact(double g[6], double A[6]) {
 }
 
 // ------------------------------------------------------------------------------------
-// LDS staging of one field of a tile
+// FP32 LDS staging of one field of a tile (the mixed form)
 // ------------------------------------------------------------------------------------
 // Smallest LDS row pitch >= bx0 (elements of esize bytes, rows of a box by rows high) at
 // which the 64 lanes of a wave, laid over the tile x fastest, then y, then z, read their
@@ -184,72 +144,45 @@ constexpr int conflict_free_pitch(int bx0, int by, int esize) {
     return bx0;
 }
 
-// Lane -> cell maps of a tile's threads. Layout 0: x fastest, then y, then z. Layout 1
-// (TX = 8, TY even, TZ a multiple of 4): lane bits 0-2 are x, bit 3 the low bit of z, bit 4
-// the low bit of y, bit 5 the second bit of z, and the wave index supplies the rest of y,
-// then of z. Unpadded rows (pitch TX + 8 = 16 doubles) then read conflict-free when a
-// plane spans 8 doubles modulo 16 (a pad of 8 doubles per plane of 192): the 16 lanes of a
-// 128-byte group of a 64-bit read are 8 x-neighbours in 2 planes (banks 0-15 and 16-31 of 32),
-// and the 32 lanes of a 256-byte group add 2 rows (banks 32-63 of 64).
-template <int TX, int TY, int TZ, int LAYOUT>
+// Lane -> cell map of the FP64 parts (16 x 4 x TZ): lane bits 0-3 are x, bit 4 the low bit of z, bit
+// 5 the low bit of y, and the wave index supplies the rest of y, then of z. A 64-bit read then
+// takes each 16-lane group from one row and the 32 lanes of two groups from two planes, which
+// are conflict-free where a plane spans 16 doubles modulo 32.
+template <int TZ>
 struct LaneMap {
-    static_assert(LAYOUT == 0 || (TX == 8 && TY % 2 == 0 && TZ % 4 == 0), "layout 1 needs 8 x even x 4k parts");
     __host__ __device__ static constexpr void cell(int tid, int& x, int& y, int& z) {
-        if (LAYOUT == 0) {
-            x = tid % TX;
-            y = (tid / TX) % TY;
-            z = tid / (TX * TY);
-        } else {
-            const int w = tid >> 6;
-            x = tid & 7;
-            z = ((tid >> 3) & 1) + 2 * ((tid >> 5) & 1) + 4 * (w / (TY / 2));
-            y = ((tid >> 4) & 1) + 2 * (w % (TY / 2));
-        }
+        const int w = tid >> 6;
+        x = tid & 15;
+        z = ((tid >> 4) & 1) + 2 * (w >> 1);
+        y = ((tid >> 5) & 1) + 2 * (w & 1);
     }
 };
 
-// whether a wave's read of its cells (elements of esize bytes, row pitch P, plane stride Q)
-// is free of bank conflicts, modelled both as 16-lane groups of 32 four-byte banks and as
-// 32-lane groups of 64 banks for 8-byte elements (64-lane groups of 64 banks for 4-byte ones)
-template <int TX, int TY, int TZ, int LAYOUT>
-constexpr bool lds_conflict_free(int P, int Q, int esize) {
-    const int words = esize / 4, NT = TX * TY * TZ;
-    for (int banks = 32; banks <= 64; banks *= 2) {
-        const int lanes = banks / words;
-        for (int base = 0; base < NT; base += lanes) {
-            bool used[64] = {};
-            for (int t = base; t < base + lanes && t < NT; ++t) {
+// whether a wave's reads of its cells (doubles, row pitch P, plane stride Q) are free of bank
+// conflicts, modelled both as 16-lane groups of 32 four-byte banks and as 32-lane groups of 64
+template <int TZ>
+constexpr bool lds_conflict_free(int P, int Q) {
+    for (int lanes = 16; lanes <= 32; lanes *= 2)
+        for (int base = 0; base < 64 * TZ; base += lanes) {
+            bool used[32] = {};
+            for (int t = base; t < base + lanes; ++t) {
                 int x = 0, y = 0, z = 0;
-                LaneMap<TX, TY, TZ, LAYOUT>::cell(t, x, y, z);
-                const int a = z * Q + y * P + x;
-                for (int w = 0; w < words; ++w) {
-                    const int bank = (a * words + w) % banks;
-                    if (used[bank]) return false;
-                    used[bank] = true;
-                }
+                LaneMap<TZ>::cell(t, x, y, z);
+                const int bank = (z * Q + y * P + x) % lanes;
+                if (used[bank]) return false;
+                used[bank] = true;
             }
         }
-    }
     return true;
 }
 
-// smallest plane stride >= P * BY that is conflict-free at row pitch P
-template <int TX, int TY, int TZ, int LAYOUT>
-constexpr int conflict_free_plane(int P, int BY, int esize) {
-    for (int q = P * BY; q < P * BY + 64; ++q)
-        if (lds_conflict_free<TX, TY, TZ, LAYOUT>(P, q, esize)) return q;
-    return P * BY;
-}
-
-template <int TX, int TY, int TZ, bool PAD = true, int ESIZE = 8, int LAYOUT = 0>
+template <int TX, int TY, int TZ, bool PAD = true>
 struct TileGeom {
     static constexpr int NT = TX * TY * TZ;
     static constexpr int BX0 = TX + 2 * HALO, BY = TY + 2 * HALO, BZ = TZ + 2 * HALO;
-    using Lanes = LaneMap<TX, TY, TZ, LAYOUT>;
-    // LDS row pitch and plane stride (elements): conflict-free centre reads
-    static constexpr int BX = (LAYOUT == 0 && GR_LDS_PAD && PAD) ? conflict_free_pitch<TX, TY>(BX0, BY, ESIZE) : BX0;
-    static constexpr int PLANE = LAYOUT == 0 ? BX * BY : conflict_free_plane<TX, TY, TZ, LAYOUT>(BX, BY, ESIZE);
-    static_assert(LAYOUT == 0 || lds_conflict_free<TX, TY, TZ, LAYOUT>(BX, PLANE, ESIZE), "no conflict-free plane");
+    // LDS row pitch and plane stride (floats): conflict-free centre reads
+    static constexpr int BX = PAD ? conflict_free_pitch<TX, TY>(BX0, BY, 4) : BX0;
+    static constexpr int PLANE = BX * BY;
     static constexpr int NLDS = PLANE * BZ;
     // sub-boxes of the halo region that some stencil reads (x0,x1,y0,y1,z0,z1)
     static constexpr int NBOX = 7;
@@ -288,93 +221,275 @@ struct TileGeom {
     }
 };
 
-// Per-thread input/output of one cell of a tile: stages the fields into LDS for the
+// LDS layout of one field's halo box of a 16 x 4 x TZ part: little more than what some stencil
+// reads. Planes z = -1 .. TZ lie one after the other in 12 rows of 24 doubles (x = -4 .. 19) and 16
+// doubles of padding, cut to rows y = -1 .. 4 on the two outer ones. Of the planes beyond (z = -4 ..
+// -2, TZ + 1 .. TZ + 3) only the z axis reads the part's own 16 x 4 columns: their rows go, two to a block
+// of 32 doubles, into the hole of the lower outer plane (A) and after the end (TE: even rows, TO:
+// odd rows), each at the place modulo 32 doubles it would have in a plane of its own, so that the
+// z taps stay free of bank conflicts. Parts of 16 x 4 x 4 take 16 KiB a field (a whole box 27) and, with the
+// rows 64-byte aligned, 158 cache lines (8 x 4 x 8 parts of the same size: 188): lines fetched into
+// the CU, not bytes from memory or arithmetic, are what a stage costs most (128^3, stages 1-2: 8x4x8
+// whole boxes 570 us, packed 535, 16x4x4 packed 508).
+template <int TZ>
+struct PackedBox {
+    static constexpr int TX = 16, TY = 4;
+    static constexpr int ROW = TX + 2 * HALO, PL = 304, NP = TZ + 2 * HALO;
+    static constexpr int LO = PL * (HALO - 1) + ROW * (HALO - 1) + HALO; // x = 0 of row y = -1 of plane z = -1
+    static constexpr int up(int e, int r) { return (e - r + 31) / 32 * 32 + r; } // next e = r modulo 32
+    static constexpr int A = up(PL * (HALO - 1) + ROW * (HALO + TY) + TX + HALO, 4);
+    static constexpr int TE = up(PL * (NP - HALO) + ROW * (HALO + TY) + TX + HALO, 4);
+    static constexpr int TO = up(TE + 5 * 32, 12);
+    static constexpr int SIZE = TO + 6 * 32 - LO;
+    static_assert(NP % 2 == 0 && PL % 32 == 16 && LO % 2 == 0, "parity of the far planes, residue of a plane");
+
+    // whether some stencil reads (x, y, z): the axes reach 4 cells, the mixed derivatives 1 on edges
+    __host__ __device__ static constexpr bool read(int x, int y, int z) {
+        const bool xi = x >= 0 && x < TX, yi = y >= 0 && y < TY, zi = z >= 0 && z < TZ;
+        const bool xe = x >= -1 && x <= TX, ye = y >= -1 && y <= TY, ze = z >= -1 && z <= TZ;
+        return (yi && zi) || (xi && zi) || (xi && yi) || (xe && ye && zi) || (xe && yi && ze) || (xi && ye && ze);
+    }
+    // planes (0, 1), (2, NP - 3), (NP - 2, NP - 1) share blocks
+    __host__ __device__ static constexpr int far(int x, int y, int p) {
+        const int j = 3 * (y >> 1) + (p < 2 ? 0 : (p >= NP - 2 ? 2 : 1));
+        const int odd = y & 1, u = (16 * p + 24 * y - 8 * odd) & 31;
+        return (odd ? TO + 32 * j : (j ? TE - 32 + 32 * j : A)) + u + x;
+    }
+    // double of the buffer that holds (x, y, z), for every point some stencil reads
+    __host__ __device__ static constexpr int pos(int x, int y, int z) {
+        const int p = z + HALO;
+        return (p < 3 || p > NP - HALO ? far(x, y, p) : PL * p + ROW * (y + HALO) + x + HALO) - LO;
+    }
+    // the point (x even) that fills double e (even) of the buffer. Doubles no stencil reads (row
+    // ends of the y halo, padding, holes) name the nearest point read of their row or the row
+    // before, so that the lane that fills them adds no cache line to its load
+    __host__ __device__ static constexpr void point(int e, int& x, int& y, int& z) {
+        e += LO;
+        const bool inA = e >= A && e < A + 32;
+        if (inA || e >= TE) {
+            const int odd = e >= TO ? 1 : 0, t = inA ? e - A : (odd ? e - TO : e - TE + 32);
+            const int b = t >> 5 > 5 ? 5 : t >> 5, h = b >= 3 ? 1 : 0, j = b - 3 * h;
+            x = t & 15;
+            y = 2 * h + odd;
+            const int half = (t >> 4) & 1, even = ((24 * y - 8 * odd) >> 4) & 1; // the half of the even plane
+            const int pe = j == 0 ? 0 : (j == 1 ? 2 : NP - 2), po = j == 0 ? 1 : (j == 1 ? NP - 3 : NP - 1);
+            z = (half == even ? pe : po) - HALO;
+            return;
+        }
+        const int pl = e / PL, r = e % PL;
+        const bool outer = pl < HALO || pl >= NP - HALO; // planes z = -1 and z = TZ
+        const int row = r / ROW - HALO, ylo = outer ? -1 : -HALO, yhi = outer ? TY : TY + HALO - 1;
+        y = row < ylo ? ylo : (row > yhi ? yhi : row);
+        z = pl > NP - HALO ? TZ : pl - HALO;
+        const bool own = y >= 0 && y < TY, edge = y >= -1 && y <= TY;
+        const int m = (own && !outer) ? HALO : ((own || (edge && !outer)) ? 2 : 0); // x reach (even)
+        x = r % ROW - HALO;
+        x = x < -m ? -m : (x > TX - 2 + m ? TX - 2 + m : x);
+    }
+    // every point read has a place of its own, in the bank of its place in a whole box, and the
+    // place knows its point
+    static constexpr bool consistent() {
+        for (int z = -HALO; z < TZ + HALO; ++z)
+            for (int y = -HALO; y < TY + HALO; ++y)
+                for (int x = -HALO; x < TX + HALO; ++x) {
+                    if (!read(x, y, z)) continue;
+                    const int e = pos(x, y, z);
+                    if (e < 0 || e >= SIZE || (e - pos(x & ~1, y, z)) != (x & 1)) return false;
+                    int u = 99, v = 99, w = 99;
+                    point(e & ~1, u, v, w);
+                    if (u != (x & ~1) || v != y || w != z) return false;
+                    const int natural = PL * (z + HALO) + ROW * (y + HALO) + x + HALO - LO;
+                    if ((e - natural) % 32 != 0) return false;
+                }
+        return true;
+    }
+};
+// Taps of a packed box: the z taps two cells off and more have an address of their own per lane.
+template <class Box>
+struct PackedTaps {
+    // the small parts run one wave per SIMD, with no other to cover a wait: all LDS reads of a field
+    // ahead of its arithmetic (a 16^3 stage 23.4 -> 21.3 us, 32^3 25.3 -> 23.4). With two waves
+    // the registers that costs are worth more (128^3: 519 us against 508 without).
+    static constexpr bool READS_FIRST = Box::NP == 2 + 2 * HALO;
+    typedef const __attribute__((address_space(3))) double* LdsPtr;
+    LdsPtr z[6]; // z - 4, - 3, - 2, + 2, + 3, + 4 in buffer 0
+    int ofs;     // first double of the current field's buffer
+    __device__ static constexpr long q(int d) {
+        return d == 0 ? 1 : (d == 1 ? Box::ROW : Box::PL);
+    }
+    __device__ __forceinline__ double at(const double* s, int d, int k) const {
+        if (d == 2 && (k >= 2 || k <= -2)) return z[k < 0 ? k + 4 : k + 1][ofs];
+        return s[k * q(d)];
+    }
+};
+
+// Per-thread input/output of one cell of an FP64 part: stages the fields into LDS for the
 // stencils (Stager interface of ccz4_cell) and combines/stores the results (Sink interface).
 //
-// Every thread owns the same NL entries of the tile's halo box for all fields, so the
-// LDS slot and the global offset of each entry are computed once. Field loads are issued
-// PF fields ahead of their use (in the fixed FIELD_ORDER), and the LDS tile is double
-// buffered: while field p is evaluated from one buffer, field p+1 is written into the
-// other, so each field costs one barrier and its HBM latency overlaps the work on the
-// fields before it. The pointwise u^n value needed by the RK3 combine of a field travels
-// with that field's prefetch.
-template <int TX, int TY, int TZ, int MODE, int PF>
-struct TileIO {
-    using T = TileGeom<TX, TY, TZ, true, 8, 0>;
-    static constexpr int NL = (T::TOTAL + T::NT - 1) / T::NT;
-    static constexpr int LBUF = T::NLDS + 1; // one LDS buffer incl. a discard slot
+// The halo goes straight from global memory to LDS, into a packed box: lane l of a wave's load of
+// chunk c writes doubles 128 c + 2 l, + 1 of the buffer, fetched from the pair of x-neighbours the
+// layout puts there (slots beyond the block fetch the part's first pair and are never read by an
+// active cell); u^n of the cells is staged beside it. With NBUF field buffers, field p + NBUF - 1 is
+// loaded while field p is evaluated. A load's LDS data is complete once the wave's vector memory
+// counter has counted it back; the counter drains in issue order (loads and stores alike), so the
+// barrier that starts field p waits until no more of this wave's operations are outstanding than it
+// has issued since the loads of field p: the loads of the fields after p stay in flight across it.
+// No vector register is loaded from memory between the first barrier and the last: the compiler does
+// not count such a load's turn among the direct ones and would drain them all at its use (nine times
+// a part when u^n went through registers).
+// The 16-byte loads are aligned to 8 bytes only where rows are of odd length.
+// UN_IN: u^n is the stage input itself (the first stage, chosen at launch), so its value at the
+// cell is the centre value the combine already receives and is not loaded again (526 us against 590
+// for the two stages of a 128^3 block, 8x4x8 parts).
+template <int TZ, int MODE, bool UN_IN>
+struct TileIODma {
+    typedef __attribute__((address_space(3))) double* LdsPtr;
+    using Box = PackedBox<TZ>;
+    static constexpr int NT = Box::TX * Box::TY * TZ;
+    static_assert(Box::consistent() && lds_conflict_free<TZ>(Box::ROW, Box::PL), "packed box of the part");
+    static constexpr int CH = 128; // doubles per chunk (64 lanes x 16 bytes)
+    static constexpr int NCH = (Box::SIZE + CH - 1) / CH;
+    static constexpr int LBUF = NCH * CH; // doubles per buffer
+    static constexpr int NW = NT / 64; // waves
+    static constexpr int KW = NCH / NW; // chunk loads per wave
+    static_assert(NT % 64 == 0 && NCH % NW == 0, "whole waves, the same number of chunks for each");
+    // doubles per buffer of the cells' own u^n values, staged beside the field (slot = thread)
+    static constexpr int UNB = MODE == MODE_RHS || UN_IN ? 0 : NT;
+    // in the last stage the new metric of every cell waits in LDS from its combine to the
+    // algebraic constraints at the end
+    static constexpr int METRIC = MODE == MODE_FINAL ? 6 * NT : 0;
+    // field buffers: as many as fit (4 at most) while two workgroups share the CU's 160 KB
+    static constexpr int fits(int n) { return (n * (LBUF + UNB) + METRIC) * 8 * 2 <= 163840; }
+    static constexpr int NBUF = fits(4) ? 4 : 3;
+    static_assert(fits(NBUF), "field buffers");
+    static constexpr int UN0 = NBUF * LBUF, METRIC0 = UN0 + NBUF * UNB; // first double of each region
+    static constexpr int LDS_DOUBLES = METRIC0 + METRIC;
+    // vector memory operations a wave issues after its loads of field `pos` and before the
+    // barrier of that field, at least: in each turn between, the loads of one more field with its
+    // u^n; for the first fields the loads issued at the start. (Results are stored too, but a
+    // wave outside the block stores none.)
+    __host__ __device__ static constexpr int younger(int pos) {
+        int n = 0;
+        for (int f = pos + 1; f <= pos + NBUF - 2 && f < NV; ++f) n += KW + (UNB && f >= NBUF - 1 ? 1 : 0);
+        return n;
+    }
 
-    double* lds; // 2 * LBUF doubles
-    const gdouble* in; // global address space: loads/stores wait on vmcnt only, never on LDS waits
+    double* lds; // LDS_DOUBLES doubles
+    const gdouble* in;
     const gdouble* un;
     gdouble* out;
     long stride;
-    long cidx;
     unsigned cb; // byte offset of the thread's cell inside one field
     int cl;
+    int wave;
     bool active;
     bool ko_on;
     StageCoef cf;
-    int loff[NL]; // LDS slot of each owned entry (T::NLDS = discard slot)
-    unsigned goff[NL]; // byte offset of the entry inside one field of the block
-    double buf[PF][NL];
-    double unb[PF];
-    double unv[NV];
-    // u^n is the stage input itself (the first stage): the u^n value of a cell is then the
-    // centre value the combine already receives, and is not loaded again (uniform)
-    bool un_in;
-    double hg[6], hA[6]; // last stage: new metric and A~ held for the algebraic constraints
+    unsigned doff[KW]; // byte offset of this lane's pair in each of its wave's chunks
+    unsigned uoff; // byte offset of the u^n pair this lane stages (lanes 0-31: the wave's 64 cells)
+    int tid;
+    PackedTaps<Box> taps;
+    double unA[6]; // u^n of A~, whose results come after the last field
+    double hA[6];
 
-    __device__ void init(int tid, int ox, int oy, int oz, int nt0, int nt1, int nt2) {
+    __device__ __forceinline__ void place(int lx, int ly, int lz) {
+        cl = Box::pos(lx, ly, lz);
 #pragma unroll
-        for (int i = 0; i < NL; ++i) {
-            const int p = tid + i * T::NT;
-            int x = 0, y = 0, z = 0;
-            T::entry(p, x, y, z);
-            const int gx = ox + x, gy = oy + y, gz = oz + z;
-            const bool ok = p < T::TOTAL && gx < nt0 && gy < nt1 && gz < nt2;
-            loff[i] = ok ? T::lds(x, y, z) : T::NLDS;
-            goff[i] = ok ? 8u * (unsigned)(gx + nt0 * (gy + nt1 * gz)) : 0u;
+        for (int k = 0; k < 6; ++k) taps.z[k] = (LdsPtr)lds + Box::pos(lx, ly, lz + (k < 3 ? k - 4 : k - 1));
+    }
+
+    // byte offset of the pair at (x, y, z) of the part, or of the part's first pair where it lies
+    // beyond the block (a pair at the end of an odd row takes the next row's first cell along)
+    __device__ __forceinline__ unsigned pair_offset(int x, int y, int z, int ox, int oy, int oz, const BlockDesc& b) const {
+        const int gx = ox + x, gy = oy + y, gz = oz + z;
+        const int i = gx + b.nt[0] * (gy + b.nt[1] * gz);
+        const bool ok = gx < b.nt[0] && gy < b.nt[1] && gz < b.nt[2] && i + 1 < b.nt[0] * b.nt[1] * b.nt[2];
+        return 8u * (unsigned)(ok ? i : ox + b.nt[0] * (oy + b.nt[1] * oz));
+    }
+
+    __device__ void init(int tid_, int ox, int oy, int oz, const BlockDesc& b) {
+        tid = tid_;
+        wave = __builtin_amdgcn_readfirstlane(tid / 64); // uniform: LDS bases go to M0 from scalars
+        const int lane = tid % 64;
+        int x = 0, y = 0, z = 0;
+#pragma unroll
+        for (int k = 0; k < KW; ++k) {
+            Box::point((wave + k * NW) * CH + 2 * lane, x, y, z);
+            doff[k] = pair_offset(x, y, z, ox, oy, oz, b);
         }
+        LaneMap<TZ>::cell(wave * 64 + 2 * (lane % 32), x, y, z);
+        uoff = pair_offset(x, y, z, ox, oy, oz, b);
 #pragma unroll
-        for (int k = 0; k < PF; ++k) prefetch(k);
-        stage_to_lds(0);
-        prefetch(PF);
+        for (int p = 0; p < NBUF - 1; ++p) prefetch(p);
     }
 
     __device__ __forceinline__ void prefetch(int pos) {
         if (pos >= NV) return;
         const int v = FIELD_ORDER[pos];
-        const int slot = pos % PF;
-        const gdouble* f = in + v * stride;
+        const gchar* f = (const gchar*)(in + v * stride);
+        // the LDS base is made opaque at every field, so the chunk addresses (M0 values) are
+        // recomputed from it with one scalar add each instead of being kept (and spilled) as
+        // 2 x KW live scalars across the whole kernel
+        unsigned base = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(LdsPtr)lds);
+#ifdef __HIP_DEVICE_COMPILE__
+        asm volatile("" : "+s"(base));
+#endif
+        LdsPtr L = (LdsPtr)(uintptr_t)base;
+        const LdsPtr U = L + UN0 + (pos % NBUF) * UNB + wave * 64;
+        L += (pos % NBUF) * LBUF;
 #pragma unroll
-        for (int i = 0; i < NL; ++i) buf[slot][i] = gload_sv(f, goff[i]);
-        if (MODE != MODE_RHS && !un_in) unb[slot] = gload(un + v * stride, cb);
+        for (int k = 0; k < KW; ++k) {
+            const int c = wave + k * NW; // uniform over the wave
+#ifdef __HIP_DEVICE_COMPILE__
+            // keeps the 32-bit offset at the load (scalar base + offset), in place
+            asm volatile("" : "+v"(doff[k]));
+#endif
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(f + doff[k]),
+                                             (__attribute__((address_space(3))) void*)(L + c * CH), 16, 0, 0);
+        }
+        // u^n of the wave's own cells (which only this wave overwrites, in the last stage)
+        if (UNB && tid % 64 < 32) {
+#ifdef __HIP_DEVICE_COMPILE__
+            asm volatile("" : "+v"(uoff));
+#endif
+            __builtin_amdgcn_global_load_lds(
+                (const __attribute__((address_space(1))) void*)((const gchar*)(un + v * stride) + uoff),
+                (__attribute__((address_space(3))) void*)U, 16, 0, 0);
+        }
+    }
+    __device__ __forceinline__ double staged_un(int v) const {
+        return lds[UN0 + (field_pos(v) % NBUF) * UNB + tid];
     }
 
-    // writes the prefetched field at position pos into its LDS buffer
-    __device__ __forceinline__ void stage_to_lds(int pos) {
-        if (pos >= NV) return;
-        const int slot = pos % PF;
-        double* L = lds + (pos & 1) * LBUF;
-#pragma unroll
-        for (int i = 0; i < NL; ++i) L[loff[i]] = buf[slot][i];
-        if (MODE != MODE_RHS && !un_in) unv[FIELD_ORDER[pos]] = unb[slot];
+    // at most n of this wave's vector memory operations outstanding (n a constant after
+    // inlining), its LDS accesses done
+    static __device__ __forceinline__ void wait_outstanding(int n) {
+#ifdef __HIP_DEVICE_COMPILE__
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"i"(n) : "memory");
+#endif
     }
-
     // ---- Stager
     __device__ double centre(int v) const { return gload(in + v * stride, cb); }
     __device__ void metric64(double g[6]) const {
 #pragma unroll
         for (int a = 0; a < 6; ++a) g[a] = gload(in + (GXX + a) * stride, cb);
     }
-    __device__ FixedStrides<1, T::BX, T::PLANE> strides() const { return {}; }
+    __device__ const PackedTaps<Box>& strides() const { return taps; }
     __device__ const double* field(int v) {
         const int pos = field_pos(v);
-        __syncthreads(); // field pos is in its buffer; every thread is done with field pos-1
-        stage_to_lds(pos + 1);
-        prefetch(pos + 1 + PF);
-        return lds + (pos & 1) * LBUF + cl;
+        // this wave's loads of field pos have landed and its LDS accesses are done; then the
+        // barrier: every wave's loads of pos have landed and every thread is done with field
+        // pos - 1, whose buffer the prefetch refills. Written as statements that may touch any
+        // memory, so the compiler keeps every access on its side; a workgroup fence would also
+        // drain the loads of the fields after pos (they write LDS)
+        wait_outstanding(younger(pos));
+#ifdef __HIP_DEVICE_COMPILE__
+        asm volatile("s_barrier" ::: "memory");
+#endif
+        prefetch(pos + NBUF - 1);
+        if (UNB && v >= AXX && v < AXX + 6) unA[v - AXX] = staged_un(v);
+        taps.ofs = (pos % NBUF) * LBUF;
+        return lds + (pos % NBUF) * LBUF + cl;
     }
 
     // ---- Sink
@@ -384,13 +499,15 @@ struct TileIO {
             if (active) gstore(out + v * stride, cb, rr);
             return;
         }
-        double val = combine_exact(cf.a1, un_in ? uin : unv[v], cf.a2, uin, cf.a3dt, rr);
+        const double u0 = UN_IN ? uin : (v >= AXX && v < AXX + 6 ? unA[v - AXX] : staged_un(v));
+        double val = combine_exact(cf.a1, u0, cf.a2, uin, cf.a3dt, rr);
         if (v == CHI) val = floor_chi(val);
         if (v == ALPHA) val = floor_alpha(val);
-        // (one wave per SIMD: the held metric costs no occupancy here, and reading it back at
-        // the end would expose a load latency)
+        // last stage: the new metric waits in LDS (this thread's own slots) for the algebraic
+        // constraints, instead of in registers across the rest of the RHS; A~ comes last and is
+        // held in registers
         if (MODE == MODE_FINAL && v >= GXX && v < GXX + 6) {
-            hg[v - GXX] = val;
+            lds[METRIC0 + (v - GXX) * NT + tid] = val;
             return;
         }
         if (MODE == MODE_FINAL && v >= AXX && v < AXX + 6) {
@@ -402,224 +519,9 @@ struct TileIO {
 
     __device__ __forceinline__ void finish() {
         if (MODE != MODE_FINAL) return;
-        algebraic_exact(hg, hA);
-        if (!active) return;
-#pragma unroll
-        for (int a = 0; a < 6; ++a) {
-            gstore(out + (GXX + a) * stride, cb, hg[a]);
-            gstore(out + (AXX + a) * stride, cb, hA[a]);
-        }
-    }
-};
-
-// TileIO whose halo staging goes straight from global memory to LDS (LDS layout 1). The
-// buffer of a field is the whole box of the part (planes of rows of TX + 8 doubles), filled
-// in 1 KiB chunks: lane l of a wave's load of chunk c writes doubles 128 c + 2 l, + 1 of the
-// buffer, fetched from the pair of x-neighbours the layout puts there (pad slots and slots
-// beyond the block fetch the field's first pair and are never read by an active cell).
-// The waves take the chunks in turn. With NBUF field buffers, field p + NBUF - 1 is loaded
-// while field p is evaluated. A load's LDS data is complete once the wave's vector memory
-// counter has counted it back; the counter drains in issue order (loads and stores alike),
-// so the barrier that starts field p waits until no more of this wave's operations are
-// outstanding than the chunk loads it has issued since those of field p: the loads of the
-// fields after p stay in flight across it.
-// Needs 16-byte aligned pairs: an even row length (nt0) and 16-byte aligned buffers.
-template <int TX, int TY, int TZ, int MODE>
-struct TileIODma {
-    typedef __attribute__((address_space(3))) double* LdsPtr;
-    using T = TileGeom<TX, TY, TZ, true, 8, 1>;
-    static constexpr int CH = 128; // doubles per chunk (64 lanes x 16 bytes)
-    static constexpr int NCH = (T::NLDS + CH - 1) / CH;
-    static constexpr int LBUF = NCH * CH; // doubles per buffer
-    static constexpr int NW = T::NT / 64; // waves
-    static constexpr int KW = (NCH + NW - 1) / NW; // chunk loads per wave
-    static_assert(T::NT % 64 == 0, "whole waves");
-    // field buffers: as many as the limit allows while two waves per SIMD (512 / NT
-    // workgroups) still share the CU's 160 KB
-    static constexpr int WG_PER_CU = 512 / T::NT;
-    static constexpr int NBUF_MAX = MODE == MODE_FINAL ? GR_DMA_BUFFERS_FINAL : GR_DMA_BUFFERS;
-    static constexpr int NBUF = (NBUF_MAX >= 3 && 3 * LBUF * 8 * WG_PER_CU <= 163840) ? 3 : 2;
-    // in the last stage also the new metric of every cell, from its combine to the
-    // algebraic constraints at the end, where it still fits beside the buffers; otherwise
-    // the metric is stored at once and read back at the end
-    static constexpr bool METRIC_LDS = MODE == MODE_FINAL && (NBUF * LBUF + 6 * T::NT) * 8 * WG_PER_CU <= 163840;
-    static constexpr int LDS_DOUBLES = NBUF * LBUF + (METRIC_LDS ? 6 * T::NT : 0);
-    // vector memory operations that every wave issues after a field's chunk loads and
-    // before the barrier of that field: the unconditional chunk loads of the next field
-    // (the last chunk of a wave may be skipped)
-    static constexpr int YOUNGER = NBUF == 3 ? KW - 1 : 0;
-    static_assert(YOUNGER < 16, "vmcnt field of s_waitcnt");
-
-    double* lds; // LDS_DOUBLES doubles
-    const gdouble* in;
-    const gdouble* un;
-    gdouble* out;
-    long stride;
-    long cidx;
-    unsigned cb;
-    int cl;
-    int wave;
-    bool active;
-    bool ko_on;
-    StageCoef cf;
-    unsigned doff[KW]; // byte offset of this lane's pair in each of its wave's chunks
-    int tid;
-    double unv[NV];
-    bool un_in; // u^n is the stage input (the first stage): not loaded again, as in TileIO
-    double hA[6];
-    // the barrier that starts a field waits for every vector memory operation issued before
-    // the chunk loads of the field after it, stores included, so a field's result is stored
-    // after the next barrier instead of just before it: the store then has a whole field to
-    // complete
-    double pend_val;
-    int pend_v;
-
-    // whether a stencil reads element x or x + 1 (x even) of row (y, z) of the box
-    __host__ __device__ static constexpr bool pair_read(int x, int y, int z) {
-        const bool zin = z >= 0 && z < TZ, zedge = z == -1 || z == TZ;
-        const bool yin = y >= 0 && y < TY, yedge = y >= -1 && y <= TY;
-        const bool xmid = x >= -2 && x <= TX, xin = x >= 0 && x < TX;
-        return zin ? (yin || xmid) : (zedge ? (yedge && xmid) : (yin && xin));
-    }
-    // pair_read against the sub-box table itself, over the whole box
-    static constexpr bool pair_read_matches_boxes() {
-        for (int z = -HALO; z < TZ + HALO; ++z)
-            for (int y = -HALO; y < TY + HALO; ++y)
-                for (int x = -HALO; x < TX + HALO; x += 2) {
-                    bool in = false;
-                    for (int b = 0; b < T::NBOX; ++b)
-                        for (int xx = x; xx <= x + 1; ++xx)
-                            in = in || (xx >= T::box[b][0] && xx < T::box[b][1] && y >= T::box[b][2] &&
-                                        y < T::box[b][3] && z >= T::box[b][4] && z < T::box[b][5]);
-                    if (in != pair_read(x, y, z)) return false;
-                }
-        return true;
-    }
-    static_assert(pair_read_matches_boxes(), "fetched rows = rows some stencil reads");
-
-    __device__ void init(int tid_, int ox, int oy, int oz, int nt0, int nt1, int nt2) {
-        tid = tid_;
-        wave = __builtin_amdgcn_readfirstlane(tid / 64); // uniform: LDS bases go to M0 from scalars
-        const int lane = tid % 64;
-#pragma unroll
-        for (int k = 0; k < KW; ++k) {
-            const int c = wave + k * NW;
-            const int e = c * CH + 2 * lane;
-            const int pl = e / T::PLANE, r = e % T::PLANE;
-            const int x = r % T::BX - HALO, y = r / T::BX - HALO, z = pl - HALO;
-            const int gx = ox + x, gy = oy + y, gz = oz + z;
-            const bool ok = c < NCH && pl < T::BZ && r < T::BX * T::BY && gx + 1 < nt0 && gy < nt1 && gz < nt2;
-            // whether a stencil reads the pair (x, x + 1) (x even): the union of the halo
-            // sub-boxes of TileGeom::box, row by row. The box corners no stencil reads (about
-            // a third of its rows) are not fetched: those lanes, and the lanes past the
-            // block, load the pair at the part's origin, a line the same field loads anyway.
-            const bool need = pair_read(x, y, z);
-            doff[k] = 8u * (unsigned)(ok && need ? gx + nt0 * (gy + nt1 * gz) : ox + nt0 * (oy + nt1 * oz));
-        }
-        pend_v = -1;
-#pragma unroll
-        for (int p = 0; p < NBUF - 1; ++p) prefetch(p);
-    }
-
-    __device__ __forceinline__ void flush() {
-        if (pend_v >= 0 && active) gstore(out + pend_v * stride, cb, pend_val);
-        pend_v = -1;
-    }
-
-    __device__ __forceinline__ void prefetch(int pos) {
-        if (pos >= NV) return;
-        const int v = FIELD_ORDER[pos];
-        const gchar* f = (const gchar*)(in + v * stride);
-        // the LDS base is made opaque at every field, so the chunk addresses (M0 values) are
-        // recomputed from it with one scalar add each instead of being kept (and spilled) as
-        // 2 x KW live scalars across the whole kernel
-        LdsPtr L = (LdsPtr)lds;
-#ifdef __HIP_DEVICE_COMPILE__
-        asm volatile("" : "+s"(L));
-#endif
-        L += (pos % NBUF) * LBUF;
-#pragma unroll
-        for (int k = 0; k < KW; ++k) {
-            const int c = wave + k * NW; // uniform over the wave
-            // every wave has chunks 0 .. KW-2; only the last may run past the box (a test on
-            // each chunk costs a lane-mask register pair per chunk, live across the kernel)
-            if (k < KW - 1 || c < NCH) {
-#ifdef __HIP_DEVICE_COMPILE__
-                // keeps the 32-bit offset at the load (scalar base + offset), in place
-                asm volatile("" : "+v"(doff[k]));
-#endif
-                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(f + doff[k]),
-                                                 (__attribute__((address_space(3))) void*)(L + c * CH), 16, 0, 0);
-            }
-        }
-        if (MODE != MODE_RHS && !un_in) unv[v] = gload(un + v * stride, cb);
-    }
-
-    // ---- Stager
-    __device__ double centre(int v) const { return gload(in + v * stride, cb); }
-    __device__ void metric64(double g[6]) const {
-#pragma unroll
-        for (int a = 0; a < 6; ++a) g[a] = gload(in + (GXX + a) * stride, cb);
-    }
-    __device__ FixedStrides<1, T::BX, T::PLANE> strides() const { return {}; }
-    __device__ const double* field(int v) {
-        const int pos = field_pos(v);
-        if (NBUF == 2) {
-            __syncthreads(); // field pos has landed in its buffer; every thread is done with pos - 1
-        } else {
-            // this wave's loads of field pos have landed (only those of pos + 1 may still be
-            // outstanding: none after the last field) and its LDS accesses are done; then
-            // the barrier: every wave's loads of pos have landed and every thread is done
-            // with field pos - 1, whose buffer the prefetch below refills. The barrier is
-            // written as a statement that may touch any memory, so the compiler keeps every
-            // access on its side of it; a workgroup fence would also drain the loads of
-            // pos + 1 (they write LDS)
-            if (pos + 1 < NV)
-                __builtin_amdgcn_s_waitcnt(0x0070 | YOUNGER); // vmcnt(YOUNGER) lgkmcnt(0)
-            else
-                __builtin_amdgcn_s_waitcnt(0x0070);
-#ifdef __HIP_DEVICE_COMPILE__
-            asm volatile("s_barrier" ::: "memory");
-#endif
-        }
-        flush();
-        prefetch(pos + NBUF - 1);
-        return lds + (pos % NBUF) * LBUF + cl;
-    }
-
-    // ---- Sink
-    __device__ __forceinline__ void put(int v, double r, double ko, double uin) {
-        const double rr = ko_on ? r + ko : r;
-        flush(); // at most one result waits (several per field only after the last barrier)
-        if (MODE == MODE_RHS) {
-            pend_v = v;
-            pend_val = rr;
-            return;
-        }
-        double val = combine_exact(cf.a1, un_in ? uin : unv[v], cf.a2, uin, cf.a3dt, rr);
-        if (v == CHI) val = floor_chi(val);
-        if (v == ALPHA) val = floor_alpha(val);
-        // last stage: the new metric waits in LDS (this thread's own slots; or in the output,
-        // read back at the end) for the algebraic constraints, instead of in registers across
-        // the rest of the RHS; A~ comes last and is held in registers
-        if (METRIC_LDS && v >= GXX && v < GXX + 6) {
-            lds[NBUF * LBUF + (v - GXX) * T::NT + tid] = val;
-            return;
-        }
-        if (MODE == MODE_FINAL && v >= AXX && v < AXX + 6) {
-            hA[v - AXX] = val;
-            return;
-        }
-        pend_v = v;
-        pend_val = val;
-    }
-
-    __device__ __forceinline__ void finish() {
-        flush();
-        if (MODE != MODE_FINAL) return;
         double hg[6];
 #pragma unroll
-        for (int a = 0; a < 6; ++a) hg[a] = METRIC_LDS ? lds[NBUF * LBUF + a * T::NT + tid] : gload(out + (GXX + a) * stride, cb);
+        for (int a = 0; a < 6; ++a) hg[a] = lds[METRIC0 + a * NT + tid];
         algebraic_exact(hg, hA);
         if (!active) return;
 #pragma unroll
@@ -630,7 +532,7 @@ struct TileIODma {
     }
 };
 
-// Mixed-precision counterpart of TileIO: the stencils and the RHS algebra see FP32
+// Mixed-precision counterpart of TileIODma: the stencils and the RHS algebra see FP32
 // values, the RK3 combine, the floors and the algebraic constraints are done in FP64 on
 // the FP64 state. Each field is staged as FP32 deltas from one FP64 reference value per
 // tile (the field at the tile's first cell): every stencil's weights sum to zero, so
@@ -640,7 +542,7 @@ struct TileIODma {
 // cell is the stage input's centre value, so it is not loaded separately
 template <int TX, int TY, int TZ, int MODE, int PF, bool UN_IN = false>
 struct TileIO32 {
-    using T = TileGeom<TX, TY, TZ, GR_LDS_PAD32 != 0, 4>;
+    using T = TileGeom<TX, TY, TZ, GR_LDS_PAD32 != 0>;
     static constexpr int NL = (T::TOTAL + T::NT - 1) / T::NT;
     static constexpr int LBUF = T::NLDS + 1;
 
@@ -859,92 +761,79 @@ __device__ __forceinline__ void load_sources(const Sources& S, long cidx, CellSo
         for (int a = 0; a < 6; ++a) src.Sij[a] = 0.0;
         return;
     }
-    src.rho = S.rho[cidx];
-    src.S = S.S[cidx];
+    const gdouble *rho = (const gdouble*)S.rho, *Si = (const gdouble*)S.Si, *Sij = (const gdouble*)S.Sij,
+                  *St = (const gdouble*)S.S;
+    src.rho = rho[cidx];
+    src.S = St[cidx];
 #pragma unroll
-    for (int a = 0; a < 3; ++a) src.Si[a] = S.Si[3 * cidx + a];
+    for (int a = 0; a < 3; ++a) src.Si[a] = Si[3 * cidx + a];
 #pragma unroll
-    for (int a = 0; a < 6; ++a) src.Sij[a] = S.Sij[6 * cidx + a];
+    for (int a = 0; a < 6; ++a) src.Sij[a] = Sij[6 * cidx + a];
 }
 
-// staging variant SV: 0 = registers into a padded box (layout 0); 1, 2 = direct LDS loads
-// into an unpadded box (layout 1); 2 runs parts twice as deep in z
-constexpr int sv_layout(int SV) { return SV == 0 ? 0 : 1; }
+static_assert(GR_TILE_X == 16 && GR_TILE_Y == 4 && GR_TILE_Z % 4 == 0, "the FP64 parts (16 x 4 x TZ) tile the launch tiles");
+constexpr int TILE_X = GR_TILE_X, TILE_Y = GR_TILE_Y, TILE_Z = GR_TILE_Z;
+// parts of a tile of TZ layers, one workgroup of 64 TZ threads each
+template <int TZ>
+constexpr int FP64_PARTS = TILE_Z / TZ;
 
-// part `part` of a tile: TX x TY x TZ cells at x = (part % (TILE_X / TX)) * TX,
-// z = (part / (TILE_X / TX)) * TZ inside the tile
-template <int TX, int TY, int TZ, int MODE, bool HAS_SRC, bool KO_EXACT, int SV>
+// part `part` of a tile: layers part * TZ .. of it
+template <int TZ, int MODE, bool HAS_SRC, bool KO_EXACT, bool UN_IN>
 __device__ __forceinline__ void stage_tile(const StageArgs& A, const TileRef& R, int part, double* lds) {
-    using T = TileGeom<TX, TY, TZ, true, 8, sv_layout(SV)>;
-    constexpr int XS = GR_TILE_X / TX;
     const BlockDesc& b = R.b;
     const int tid = threadIdx.x;
     int lx = 0, ly = 0, lz = 0;
-    T::Lanes::cell(tid, lx, ly, lz);
-    const int x0 = R.tix * GR_TILE_X + (part % XS) * TX;
-    const int z0 = R.tiz * GR_TILE_Z + (part / XS) * TZ;
-    const int ix = x0 + lx, iy = R.tiy * TY + ly, iz = z0 + lz; // interior-relative
+    LaneMap<TZ>::cell(tid, lx, ly, lz);
+    const int x0 = R.tix * TILE_X, y0 = R.tiy * TILE_Y, z0 = R.tiz * TILE_Z + part * TZ;
+    const int ix = x0 + lx, iy = y0 + ly, iz = z0 + lz; // interior-relative
     const bool active = ix < b.n[0] && iy < b.n[1] && iz < b.n[2];
     const int gi = b.ng + (active ? ix : 0), gj = b.ng + (active ? iy : 0), gk = b.ng + (active ? iz : 0);
     const long cidx = gi + (long)b.nt[0] * (gj + (long)b.nt[1] * gk);
 
-    typename std::conditional<SV != 0, TileIODma<TX, TY, TZ, MODE>, TileIO<TX, TY, TZ, MODE, GR_FP64_PREFETCH>>::type io;
+    TileIODma<TZ, MODE, UN_IN> io;
     io.lds = lds;
     io.in = R.in;
     io.un = R.un;
-    io.un_in = R.un == R.in;
     io.out = R.out;
     io.stride = b.stride;
-    io.cidx = cidx;
     io.cb = 8u * (unsigned)cidx;
-    io.cl = T::lds(lx, ly, lz);
+    io.place(lx, ly, lz);
     io.active = active;
     io.ko_on = A.ko_on != 0;
     io.cf = A.cf;
-    io.init(tid, b.ng + x0, b.ng + R.tiy * TY, b.ng + z0, b.nt[0], b.nt[1], b.nt[2]);
+    io.init(tid, b.ng + x0, b.ng + y0, b.ng + z0, b);
 
     CellSources src{};
     if (HAS_SRC) load_sources(R.src, cidx, src);
     ccz4_cell<double, HAS_SRC, KO_EXACT>(io, io, A.K, A.P, src);
 }
 
-// parts of a tile of TX x . x TZ cells
-template <int TX, int TZ>
-constexpr int parts_of() { return (GR_TILE_X / TX) * (GR_TILE_Z / TZ); }
-
-// LDS doubles of one FP64 part's two field buffers under staging variant SV
-template <int TX, int TY, int TZ, int SV, int MODE>
-constexpr int fp64_lds_doubles() {
-    return SV != 0 ? TileIODma<TX, TY, TZ, MODE>::LDS_DOUBLES : 2 * (TileGeom<TX, TY, TZ, true, 8, 0>::NLDS + 1);
-}
-
 // whether part `part` of tile R holds no cell of the block (uniform over the workgroup)
-template <int TX, int TZ>
+template <int TZ>
 __device__ __forceinline__ bool part_outside(const TileRef& R, int part) {
-    constexpr int XS = GR_TILE_X / TX;
-    return R.tix * GR_TILE_X + (part % XS) * TX >= R.b.n[0] || R.tiz * GR_TILE_Z + (part / XS) * TZ >= R.b.n[2];
+    return R.tiz * TILE_Z + part * TZ >= R.b.n[2];
 }
 
-// one part of one tile per workgroup (parts_of consecutive workgroups per tile)
-template <int TX, int TY, int TZ, int MODE, bool HAS_SRC, bool KO_EXACT, int SV>
-__global__ __launch_bounds__(TX* TY* TZ, GR_FP64_MIN_WAVES) void stage_kernel(StageArgs A) {
-    constexpr int NP = parts_of<TX, TZ>();
-    __shared__ double lds[fp64_lds_doubles<TX, TY, TZ, SV, MODE>()];
+// one part of one tile per workgroup (FP64_PARTS consecutive workgroups per tile); two waves per
+// SIMD (256 registers) for the large parts
+template <int TZ, int MODE, bool HAS_SRC, bool KO_EXACT, bool UN_IN>
+__global__ __launch_bounds__(64 * TZ, TZ / 2) void stage_kernel(StageArgs A) {
+    constexpr int NP = FP64_PARTS<TZ>;
+    __shared__ __align__(16) double lds[TileIODma<TZ, MODE, UN_IN>::LDS_DOUBLES];
     const int slot = tile_of_block(blockIdx.x, A.ntiles * NP, A.xcd_remap);
     const int tile = slot / NP, part = slot % NP;
-    if (A.flags && A.flags[tile] != A.want) return; // whole workgroup leaves before any barrier
     const TileRef R = resolve_tile(A, tile);
-    if (part_outside<TX, TZ>(R, part)) return;
-    stage_tile<TX, TY, TZ, MODE, HAS_SRC, KO_EXACT, SV>(A, R, part, lds);
+    if (part_outside<TZ>(R, part)) return; // whole workgroup leaves before any barrier
+    stage_tile<TZ, MODE, HAS_SRC, KO_EXACT, UN_IN>(A, R, part, lds);
 }
 
 // the flagged tiles only, from a small grid: each workgroup gathers the tiles with
 // flags == want among tiles blockIdx.x + k * gridDim.x and runs them one after the other
 // (every thread takes the same trip counts, so the barriers are uniform)
-template <int TX, int TY, int TZ, int MODE, bool HAS_SRC, bool KO_EXACT, int SV>
-__global__ __launch_bounds__(TX* TY* TZ, GR_FP64_MIN_WAVES) void stage_kernel_scan(StageArgs A) {
-    constexpr int NT = TX * TY * TZ;
-    __shared__ double lds[fp64_lds_doubles<TX, TY, TZ, SV, MODE>()];
+template <int TZ, int MODE, bool HAS_SRC, bool KO_EXACT, bool UN_IN>
+__global__ __launch_bounds__(64 * TZ) void stage_kernel_scan(StageArgs A) {
+    constexpr int NT = 64 * TZ;
+    __shared__ __align__(16) double lds[TileIODma<TZ, MODE, UN_IN>::LDS_DOUBLES];
     __shared__ int list[NT];
     __shared__ int nlist;
     const int per = (int)gridDim.x * NT;
@@ -958,41 +847,30 @@ __global__ __launch_bounds__(TX* TY* TZ, GR_FP64_MIN_WAVES) void stage_kernel_sc
         __syncthreads();
         for (int item = 0; item < n; ++item) {
             const TileRef R = resolve_tile(A, list[item]);
-            for (int part = 0; part < parts_of<TX, TZ>(); ++part) {
-                if (part_outside<TX, TZ>(R, part)) continue; // uniform over the workgroup
-                stage_tile<TX, TY, TZ, MODE, HAS_SRC, KO_EXACT, SV>(A, R, part, lds);
+            for (int part = 0; part < FP64_PARTS<TZ>; ++part) {
+                if (part_outside<TZ>(R, part)) continue; // uniform over the workgroup
+                stage_tile<TZ, MODE, HAS_SRC, KO_EXACT, UN_IN>(A, R, part, lds);
                 __syncthreads(); // the next part reuses the LDS buffers
             }
         }
     }
 }
 
-static_assert(GR_TILE_X % GR_FP64_SPLIT == 0 && GR_TILE_Z % GR_FP64_ZSPLIT == 0,
-              "the FP64 split must divide the tile");
-constexpr int TILE_X = GR_TILE_X, TILE_Y = GR_TILE_Y, TILE_Z = GR_TILE_Z;
-constexpr int FP64_TX = GR_TILE_X / GR_FP64_SPLIT, FP64_TY = GR_TILE_Y, FP64_TZ = GR_TILE_Z / GR_FP64_ZSPLIT;
-static_assert(!GR_LDS_PAD || FP64_TX != 8 || TILE_X != 16 || TILE_Y != 4 ||
-                  (TileGeom<FP64_TX, FP64_TY, FP64_TZ, true, 8, 1>::BX == 16 &&
-                   TileGeom<FP64_TX, FP64_TY, FP64_TZ, true, 8, 1>::PLANE == 200 &&
-                   TileGeom<FP64_TX, FP64_TY, FP64_TZ>::BX == 24 && TileGeom<TILE_X, TILE_Y, TILE_Z, true, 4>::BX == 48),
-              "LDS layouts of the default tiles: FP64 rows of 24 (layout 0), rows of 16 in planes of 200 (layout "
-              "1); FP32 rows of 48");
-// part shapes of the staging variants: 0 and 1 the build's part, 2 twice as deep in z
-template <int SV>
-struct SvShape {
-    static constexpr int TX = SV == 0 ? FP64_TX : 8, TY = SV == 0 ? FP64_TY : 4, TZ = SV == 0 ? FP64_TZ : (SV == 1 ? 4 : 8);
-    static constexpr int NT = TX * TY * TZ, PARTS = parts_of<TX, TZ>();
-};
-static_assert(TILE_X == 16 && TILE_Y == 4 && TILE_Z == 8, "the direct-staging parts (8x4x4, 8x4x8) tile 16x4x8 tiles");
-static_assert(FP64_STAGE_VARIANTS == 3, "staging variants 0, 1, 2");
-// workgroups of the FP64 pass of the mixed form: 256 threads per CU
-constexpr int FP64_SCAN_GRID = 256 * 256 / (FP64_TX * FP64_TY * FP64_TZ);
+// Layers of the parts of large and of small launches, and the tiles from which a launch is large.
+// Larger parts load less halo per cell; a launch whose small parts find a CU each takes as long
+// as one part, and a small part is the shorter (stages 1-2 / 3, us, 2 against 4 layers: 16^3
+// 21.3 / 23.0 against 23.9 / 24.9, 32^3, 64 tiles, 23.4 / 25.5 against 25.2 / 26.7; 37x29x23, 72
+// tiles, 29.2 / 25.8 against 25.1 / 26.2).
+constexpr int TZ_LARGE = 4, TZ_SMALL = 2;
+constexpr int LARGE_TILES = 256 / FP64_PARTS<TZ_SMALL> + 1; // small parts outnumber the 256 CUs
+// workgroups of the FP64 pass of the mixed form: one per CU
+constexpr int FP64_SCAN_GRID = 256;
 
 // one part of TX x TY x TZ cells (TILE_X / TX parts along x) of a launch tile per workgroup;
 // the tile is the unit of the FP32 / FP64 choice
 template <int TX, int TY, int TZ, int MODE, bool HAS_SRC, bool UN_IN = false>
 __global__ __launch_bounds__(TX* TY* TZ, GR_MIXED_MIN_WAVES) void stage_kernel_mixed(StageArgs A) {
-    using T = TileGeom<TX, TY, TZ, GR_LDS_PAD32 != 0, 4>;
+    using T = TileGeom<TX, TY, TZ, GR_LDS_PAD32 != 0>;
     constexpr int NP = GR_TILE_X / TX;
     static_assert(GR_TILE_X % TX == 0 && TY == GR_TILE_Y && TZ == GR_TILE_Z, "parts split the tile along x");
     __shared__ float lds[2 * (T::NLDS + 1)];
@@ -1052,24 +930,26 @@ __global__ __launch_bounds__(TX* TY* TZ) void classify_tiles_kernel(StageArgs A,
     if (tid == 0) flags[tile] = (unsigned char)bad;
 }
 
-// scan: nblk workgroups gather the flagged tiles; otherwise one workgroup per part
-template <int MODE, bool HAS_SRC, int SV>
-hipError_t launch_stage_sv(const StageArgs& A, int scan_grid, hipStream_t s) {
-    using S = SvShape<SV>;
-    if (A.scan)
-        stage_kernel_scan<S::TX, S::TY, S::TZ, MODE, HAS_SRC, GR_FP64_KO_EXACT != 0, SV>
-            <<<dim3(scan_grid), dim3(S::NT), 0, s>>>(A);
+template <int MODE, bool HAS_SRC, bool UN_IN>
+hipError_t launch_stage_form(const StageArgs& A, int scan_grid, bool large, hipStream_t s) {
+    constexpr bool KO = GR_FP64_KO_EXACT != 0;
+    if (A.scan) // the flagged tiles, gathered by a small grid
+        stage_kernel_scan<TZ_LARGE, MODE, HAS_SRC, KO, UN_IN><<<dim3(scan_grid), dim3(64 * TZ_LARGE), 0, s>>>(A);
+    else if (A.ntiles > 0 && large)
+        stage_kernel<TZ_LARGE, MODE, HAS_SRC, KO, UN_IN>
+            <<<dim3(A.ntiles * FP64_PARTS<TZ_LARGE>), dim3(64 * TZ_LARGE), 0, s>>>(A);
     else if (A.ntiles > 0)
-        stage_kernel<S::TX, S::TY, S::TZ, MODE, HAS_SRC, GR_FP64_KO_EXACT != 0, SV>
-            <<<dim3(A.ntiles * S::PARTS), dim3(S::NT), 0, s>>>(A);
+        stage_kernel<TZ_SMALL, MODE, HAS_SRC, KO, UN_IN>
+            <<<dim3(A.ntiles * FP64_PARTS<TZ_SMALL>), dim3(64 * TZ_SMALL), 0, s>>>(A);
     return hipGetLastError();
 }
 
 template <int MODE, bool HAS_SRC>
-hipError_t launch_stage_t(const StageArgs& A, int scan_grid, int variant, hipStream_t s) {
-    if (variant == 1) return launch_stage_sv<MODE, HAS_SRC, 1>(A, scan_grid, s);
-    if (variant == 2) return launch_stage_sv<MODE, HAS_SRC, 2>(A, scan_grid, s);
-    return launch_stage_sv<MODE, HAS_SRC, 0>(A, scan_grid, s);
+hipError_t launch_stage_t(const StageArgs& A, int scan_grid, bool large, hipStream_t s) {
+    // the first stage (u^n is the stage input) has an instance of its own: no u^n loads
+    if (MODE == MODE_STAGE && A.sel_un == A.sel_in)
+        return launch_stage_form<MODE, HAS_SRC, MODE == MODE_STAGE>(A, scan_grid, large, s);
+    return launch_stage_form<MODE, HAS_SRC, false>(A, scan_grid, large, s);
 }
 
 // ------------------------------------------------------------------------------------
@@ -1402,7 +1282,7 @@ __global__ void dissipation_kernel(BlockDesc b, const double* __restrict__ u, do
         const double* f = u + v * b.stride + c;
         double acc = 0.0;
         for (int d = 0; d < 3; ++d)
-            acc = ko_axis_ordered(acc, K.kw[d], f[-3 * st[d]], f[-2 * st[d]], f[-st[d]], f[0], f[st[d]], f[2 * st[d]],
+            acc = ko_axis_ordered(d == 0, acc, K.kw[d], f[-3 * st[d]], f[-2 * st[d]], f[-st[d]], f[0], f[st[d]], f[2 * st[d]],
                                   f[3 * st[d]]);
         rhs[v * b.stride + c] += acc;
     }
@@ -1843,9 +1723,9 @@ Stencil<double> make_stencil(const BlockDesc& b, double ko_sigma) {
 }
 
 void stage_tile_fp64(int* t3) {
-    t3[0] = FP64_TX;
-    t3[1] = FP64_TY;
-    t3[2] = FP64_TZ;
+    t3[0] = TILE_X;
+    t3[1] = TILE_Y;
+    t3[2] = TZ_LARGE;
 }
 
 void stage_tile_mixed(int* t3) {
@@ -1945,8 +1825,7 @@ Batch single_batch(const BlockDesc& b, const double* in, const double* un, doubl
 hipError_t launch_stage_fp64(const Batch& B, const int sel[3], bool has_src, const CellParams& P,
                              double ko_sigma, int mode, const StageCoef& cf, hipStream_t s,
                              const unsigned char* flags) {
-    // the direct LDS staging reads 16-byte pairs: other batches run the register staging
-    const int variant = (B.variant != 0 && B.pairs_ok) ? B.variant : 0;
+    const bool large = B.variant == 2 || (B.variant == 0 && B.ntiles >= LARGE_TILES);
     StageArgs A = stage_args(B, sel, P, ko_sigma, cf, flags, 1);
     // with flags (the FP64 tiles of the mixed form: few, near the puncture) a small grid
     // gathers them instead of launching one workgroup per part of every tile of the level
@@ -1956,13 +1835,13 @@ hipError_t launch_stage_fp64(const Batch& B, const int sel[3], bool has_src, con
         nblk = A.ntiles < FP64_SCAN_GRID ? A.ntiles : FP64_SCAN_GRID;
     }
     if (has_src) {
-        if (mode == MODE_RHS) return launch_stage_t<MODE_RHS, true>(A, nblk, variant, s);
-        if (mode == MODE_STAGE) return launch_stage_t<MODE_STAGE, true>(A, nblk, variant, s);
-        return launch_stage_t<MODE_FINAL, true>(A, nblk, variant, s);
+        if (mode == MODE_RHS) return launch_stage_t<MODE_RHS, true>(A, nblk, large, s);
+        if (mode == MODE_STAGE) return launch_stage_t<MODE_STAGE, true>(A, nblk, large, s);
+        return launch_stage_t<MODE_FINAL, true>(A, nblk, large, s);
     }
-    if (mode == MODE_RHS) return launch_stage_t<MODE_RHS, false>(A, nblk, variant, s);
-    if (mode == MODE_STAGE) return launch_stage_t<MODE_STAGE, false>(A, nblk, variant, s);
-    return launch_stage_t<MODE_FINAL, false>(A, nblk, variant, s);
+    if (mode == MODE_RHS) return launch_stage_t<MODE_RHS, false>(A, nblk, large, s);
+    if (mode == MODE_STAGE) return launch_stage_t<MODE_STAGE, false>(A, nblk, large, s);
+    return launch_stage_t<MODE_FINAL, false>(A, nblk, large, s);
 }
 
 template <int MODE, bool HAS_SRC>

@@ -51,10 +51,8 @@ constexpr int GHOST_WG = 256;
 // workgroup w; each block's ghost cells start on a workgroup of their own) or the single
 // block `one`. sel_* pick the buffer of
 // each block that is the stage input, u^n and the output (0, 1, 2 = buf[0..2]).
-// FP64 staging variants of the stage kernel (chosen per launch, by the autotuner): 0 = halo
-// prefetched into registers and written to a padded LDS box (parts of 8x4x4 cells, one wave
-// per SIMD); 1 = halo loaded straight into an unpadded LDS box (8x4x4, two waves per SIMD);
-// 2 = as 1 with parts of 8x4x8 (less halo per cell). 1 and 2 need even row lengths.
+// FP64 forms of the stage kernel (chosen per launch, by the autotuner): 0 = parts of 16x4x2 or
+// 16x4x4 cells by the size of the launch, 1 = always 16x4x2, 2 = always 16x4x4.
 constexpr int FP64_STAGE_VARIANTS = 3;
 
 struct Batch {
@@ -66,11 +64,11 @@ struct Batch {
     int ntiles;
     int ghost_wgs; // workgroups of a ghost launch
     double dx[3]; // grid spacing shared by all blocks of the launch
-    int pairs_ok; // every block: even row length (nt0) and 16-byte aligned buffers
-    int variant;  // FP64 staging variant (0 registers, 1 direct LDS; 1 needs pairs_ok)
+    int pairs_ok; // every block: even row length (nt0) and 16-byte aligned buffers (forms 1, 2)
+    int variant;  // FP64 form of the stage kernel
     int ghost_groups; // field groups of the ghost fill launch (1, 2, 4 or 11)
 };
-// whether block b's rows can be read as 16-byte pairs from buffer p
+// whether block b's rows can be read as aligned 16-byte pairs from buffer p
 bool pairs_aligned(const BlockDesc& b, const void* p);
 
 // builds the tile bookkeeping of a block list (host side): tile0/tiles and ghost_wg0 of

@@ -323,10 +323,9 @@ int gr_level_profile_read(gr_level* lvl, int kind, double* total_ms, int* launch
 /* ---- autotuning (no reference counterpart: the reference's only schedule is a fixed OpenMP
  * collapse(3) schedule(static), src/spacetime/ccz4.cpp:266-268) ---------------------------- */
 
-/* Tuned choices. GR_TUNE_STAGE: the FP64 stage kernel's halo staging, 0 = prefetch through
- * registers into a padded LDS box (8x4x4-cell parts, one wave per SIMD), 1 = direct
- * global-to-LDS loads into an unpadded box (8x4x4, two waves per SIMD), 2 = as 1 with
- * 8x4x8-cell parts (less halo per cell); 1 and 2 need even row lengths (others run 0).
+/* Tuned choices. GR_TUNE_STAGE: the parts of a launch tile the FP64 stage kernel's workgroups run,
+ * 0 = 16x4x2 or 16x4x4 cells by the size of the launch, 1 = always 16x4x2, 2 = always 16x4x4 (less
+ * halo per cell); 1 and 2 need even row lengths (others run 0).
  * GR_TUNE_GHOST / GR_TUNE_TRANSFER: field groups (1, 2, 4 or 11) of the ghost fill and of the
  * prolongation and restriction launches. */
 enum gr_tune_kind { GR_TUNE_STAGE = 0, GR_TUNE_GHOST = 1, GR_TUNE_TRANSFER = 2 };
@@ -354,7 +353,7 @@ int gr_hierarchy_get_tuning(gr_hierarchy* h, int level, int* groups);
 int gr_hierarchy_set_tuning(gr_hierarchy* h, int level, int groups);
 /* The process-wide tuning table: write to / read from a text file (one line per entry:
  * kind class precision value), or empty it. Levels and hierarchies created afterwards use
- * the entries of their class; absent entries keep the defaults (staging 2 for a group of
+ * the entries of their class; absent entries keep the defaults (stage form 2 for a group of
  * blocks with even row lengths and at least 40^3 interior cells in all, else 0; 4 groups). */
 int gr_tune_save(const char* path);
 int gr_tune_load(const char* path);
