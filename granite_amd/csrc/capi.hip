@@ -80,11 +80,8 @@ struct gr_level {
     std::vector<double*> u, s1, s2;
     std::vector<gr::Sources> src;   // per block (device pointers borrowed from the caller)
     bool has_src = false;
-    double* ham = nullptr;     // monitor scratch (max stride)
-    double* mom = nullptr;     // momentum-constraint scratch (3 * max stride, on first use)
-    long maxstride = 0;
-    double* partial = nullptr; // reduction partials
-    double* red = nullptr;     // reduction result (1 double)
+    double* partial = nullptr; // reduction partials (2 * partial_cap doubles)
+    double* red = nullptr;     // reduction results (2 doubles per block)
     double* cfl_part = nullptr; // CFL-guard partials and result (on first use)
     double* bh = nullptr;      // puncture masses/positions for initial data
     double chi_fp64_below = 0.2;
@@ -499,7 +496,6 @@ int gr_level_create(gr_engine* e, int nblocks, const gr_geom* geoms, gr_level** 
     *out = nullptr;
     gr_level* L = new gr_level();
     L->eng = e;
-    long maxstride = 0;
     for (int i = 0; i < nblocks; ++i) {
         gr::BlockDesc b;
         if ((rc = check_geom(e, &geoms[i], &b))) {
@@ -507,7 +503,6 @@ int gr_level_create(gr_engine* e, int nblocks, const gr_geom* geoms, gr_level** 
             return rc;
         }
         L->blk.push_back(b);
-        if (b.stride > maxstride) maxstride = b.stride;
         double *u = nullptr, *a = nullptr, *c = nullptr;
         hipError_t st = alloc_state(b, &u);
         if (st == hipSuccess) st = alloc_state(b, &a);
@@ -554,10 +549,8 @@ int gr_level_create(gr_engine* e, int nblocks, const gr_geom* geoms, gr_level** 
         int g = 0;
         if (tune_get(GR_TUNE_GHOST, level_class(L), GR_PREC_FP64, &g)) L->batch.ghost_groups = g;
     }
-    L->maxstride = maxstride;
-    if (st == hipSuccess) st = hipMalloc((void**)&L->ham, maxstride * sizeof(double));
-    if (st == hipSuccess) st = hipMalloc((void**)&L->partial, L->partial_cap * sizeof(double));
-    if (st == hipSuccess) st = hipMalloc((void**)&L->red, sizeof(double));
+    if (st == hipSuccess) st = hipMalloc((void**)&L->partial, 2 * L->partial_cap * sizeof(double));
+    if (st == hipSuccess) st = hipMalloc((void**)&L->red, 2 * L->blk.size() * sizeof(double));
     if (st != hipSuccess) {
         gr_level_destroy(L);
         return hipfail(e, st, "hipMalloc(level scratch)");
@@ -598,8 +591,6 @@ int gr_level_destroy(gr_level* L) {
     if (L->d_table) (void)hipFree(L->d_table);
     if (L->d_tile_block) (void)hipFree(L->d_tile_block);
     if (L->d_ghost_wg_block) (void)hipFree(L->d_ghost_wg_block);
-    if (L->ham) (void)hipFree(L->ham);
-    if (L->mom) (void)hipFree(L->mom);
     if (L->partial) (void)hipFree(L->partial);
     if (L->red) (void)hipFree(L->red);
     if (L->cfl_part) (void)hipFree(L->cfl_part);
@@ -998,28 +989,39 @@ int gr_level_sync(gr_level* L) {
     return gr_engine_sync(L->eng);
 }
 
+} // extern "C"
+
+// the constraint sums of every block of a level and their copy to `h` (per block, with_mom: H^2
+// and |M|^2), in stream order; h is complete after the next synchronisation
+static hipError_t enqueue_monitor(gr_level* L, bool with_mom, std::vector<double>& h) {
+    hipStream_t s = L->eng->stream;
+    const size_t k = with_mom ? 2 : 1;
+    h.assign(k * L->blk.size(), 0.0);
+    for (size_t b = 0; b < L->blk.size(); ++b) {
+        const hipError_t st = gr::launch_constraint_sums(L->blk[b], L->u[b], with_mom, L->partial, L->partial_cap,
+                                                         L->red + k * b, s);
+        if (st != hipSuccess) return st;
+    }
+    return hipMemcpyAsync(h.data(), L->red, h.size() * sizeof(double), hipMemcpyDeviceToHost, s);
+}
+
+extern "C" {
+
 int gr_level_constraints_l2(gr_level* L, double* sumsq, long long* count) {
     if (!L) return GR_ERR_ARG;
     gr_engine* e = L->eng;
     int rc = use_device(e);
     if (rc) return rc;
     if (!sumsq || !count) return fail(e, GR_ERR_ARG, "null output");
-    double total = 0.0;
-    long long n = 0;
+    std::vector<double> h;
+    GR_HIP(e, enqueue_monitor(L, false, h));
+    GR_HIP(e, hipStreamSynchronize(e->stream));
+    *sumsq = 0.0;
+    *count = 0;
     for (size_t b = 0; b < L->blk.size(); ++b) {
-        const gr::BlockDesc& B = L->blk[b];
-        int nparts = 0;
-        GR_HIP(e, gr::launch_constraints(B, L->u[b], L->ham, nullptr, e->stream));
-        GR_HIP(e, gr::launch_sumsq_interior(B, L->ham, 1, L->partial, L->partial_cap, &nparts, e->stream));
-        GR_HIP(e, gr::launch_sum_partials(L->partial, nparts, L->red, e->stream));
-        double h = 0.0;
-        GR_HIP(e, hipMemcpyAsync(&h, L->red, sizeof(double), hipMemcpyDeviceToHost, e->stream));
-        GR_HIP(e, hipStreamSynchronize(e->stream));
-        total += h;
-        n += (long long)B.n[0] * B.n[1] * B.n[2];
+        *sumsq += h[b];
+        *count += (long long)L->blk[b].n[0] * L->blk[b].n[1] * L->blk[b].n[2];
     }
-    *sumsq = total;
-    *count = n;
     return GR_OK;
 }
 
@@ -1031,13 +1033,7 @@ int gr_ccz4_constraints_l2_noalloc(gr_engine* e, const gr_geom* geom, const doub
     if ((rc = check_geom(e, geom, &b))) return rc;
     if (!d_u || !d_sumsq || !count) return fail(e, GR_ERR_ARG, "null state or output");
     if (!e->scratch) return fail(e, GR_ERR_NODEV, "no scratch address on this device");
-    // the partition gives each workgroup at least ceil(cells / kNoAllocPartials) cells, so
-    // every block the geometry check accepts fits the scratch; checked before any launch
-    if (gr::reduce_parts(b, kNoAllocPartials) > kNoAllocPartials)
-        return fail(e, GR_ERR_GEOM, "block needs more reduction partials than the scratch holds (2048)");
-    int nparts = 0;
-    GR_HIP(e, gr::launch_ham_sumsq(b, d_u, e->scratch, kNoAllocPartials, &nparts, e->stream));
-    GR_HIP(e, gr::launch_sum_partials(e->scratch, nparts, d_sumsq, e->stream));
+    GR_HIP(e, gr::launch_constraint_sums(b, d_u, false, e->scratch, kNoAllocPartials, d_sumsq, e->stream));
     *count = (long long)b.n[0] * b.n[1] * b.n[2];
     return GR_OK;
 }
@@ -1061,16 +1057,16 @@ int gr_level_nonfinite(gr_level* L, long long* count) {
     int rc = use_device(e);
     if (rc) return rc;
     if (!count) return fail(e, GR_ERR_ARG, "null output");
-    double total = 0.0;
+    std::vector<double> h(L->blk.size());
     for (size_t b = 0; b < L->blk.size(); ++b) {
         int nparts = 0;
         GR_HIP(e, gr::launch_count_nonfinite(L->blk[b], L->u[b], L->partial, L->partial_cap, &nparts, e->stream));
-        GR_HIP(e, gr::launch_sum_partials(L->partial, nparts, L->red, e->stream));
-        double h = 0.0;
-        GR_HIP(e, hipMemcpyAsync(&h, L->red, sizeof(double), hipMemcpyDeviceToHost, e->stream));
-        GR_HIP(e, hipStreamSynchronize(e->stream));
-        total += h;
+        GR_HIP(e, gr::launch_sum_partials(L->partial, nparts, L->red + b, e->stream));
     }
+    GR_HIP(e, hipMemcpyAsync(h.data(), L->red, h.size() * sizeof(double), hipMemcpyDeviceToHost, e->stream));
+    GR_HIP(e, hipStreamSynchronize(e->stream));
+    double total = 0.0;
+    for (double v : h) total += v;
     *count = (long long)total;
     return GR_OK;
 }
@@ -1635,28 +1631,22 @@ int gr_hierarchy_constraints_l2(gr_hierarchy* H, double* ham_sumsq, double* mom_
     int rc = use_device(e);
     if (rc) return rc;
     if (!count) return fail(e, GR_ERR_ARG, "null output");
+    const bool with_mom = mom_sumsq != nullptr;
+    std::vector<std::vector<double>> h(H->lv.size());
+    hipError_t st = hipSuccess;
+    for (size_t l = 0; l < H->lv.size() && st == hipSuccess; ++l) st = enqueue_monitor(H->lv[l], with_mom, h[l]);
+    const hipError_t done = hipStreamSynchronize(e->stream); // also before h goes, where a level failed
+    if (st == hipSuccess) st = done;
+    if (st != hipSuccess) return hipfail(e, st, "constraint monitor");
     double th = 0.0, tm = 0.0;
     long long n = 0;
-    for (gr_level* L : H->lv) {
-        if (mom_sumsq && !L->mom) GR_HIP(e, hipMalloc((void**)&L->mom, 3 * L->maxstride * sizeof(double)));
-        for (size_t b = 0; b < L->blk.size(); ++b) {
-            const gr::BlockDesc& B = L->blk[b];
-            GR_HIP(e, gr::launch_constraints(B, L->u[b], L->ham, mom_sumsq ? L->mom : nullptr, e->stream));
-            double h[2] = {0.0, 0.0};
-            for (int q = 0; q < 2; ++q) {
-                if (q == 0 ? !ham_sumsq : !mom_sumsq) continue;
-                int nparts = 0;
-                GR_HIP(e, gr::launch_sumsq_interior(B, q == 0 ? L->ham : L->mom, q == 0 ? 1 : 3, L->partial,
-                                                    L->partial_cap, &nparts, e->stream));
-                GR_HIP(e, gr::launch_sum_partials(L->partial, nparts, L->red, e->stream));
-                GR_HIP(e, hipMemcpyAsync(&h[q], L->red, sizeof(double), hipMemcpyDeviceToHost, e->stream));
-                GR_HIP(e, hipStreamSynchronize(e->stream));
-            }
-            th += h[0];
-            tm += h[1];
+    for (size_t l = 0; l < H->lv.size(); ++l)
+        for (size_t b = 0; b < H->lv[l]->blk.size(); ++b) {
+            const gr::BlockDesc& B = H->lv[l]->blk[b];
+            th += h[l][with_mom ? 2 * b : b];
+            if (with_mom) tm += h[l][2 * b + 1];
             n += (long long)B.n[0] * B.n[1] * B.n[2];
         }
-    }
     if (ham_sumsq) *ham_sumsq = th;
     if (mom_sumsq) *mom_sumsq = tm;
     *count = n;

@@ -323,6 +323,26 @@ struct PackedTaps {
     }
 };
 
+// Order in which a kernel stages the fields: N fields, field(pos) at position pos.
+struct RhsOrder {
+    static constexpr int N = NV;
+    __host__ __device__ static constexpr int field(int pos) { return FIELD_ORDER[pos]; }
+    __host__ __device__ static constexpr int pos(int v) { return field_pos(v); }
+};
+// The constraint monitor's: metric, chi, Gamma-hat for H; with the momentum constraint also K and A~.
+template <bool MOM>
+struct MonitorOrder {
+    static constexpr int N = MOM ? 17 : 10;
+    __host__ __device__ static constexpr int field(int pos) {
+        return pos < 6 ? GXX + pos : (pos == 6 ? CHI : (pos < 10 ? GHX + pos - 7 : (pos == 10 ? KTR : AXX + pos - 11)));
+    }
+    __host__ __device__ static constexpr int pos(int v) {
+        int p = 0;
+        while (field(p) != v) ++p;
+        return p;
+    }
+};
+
 // Per-thread input/output of one cell of an FP64 part: stages the fields into LDS for the
 // stencils (Stager interface of ccz4_cell) and combines/stores the results (Sink interface).
 //
@@ -341,7 +361,7 @@ struct PackedTaps {
 // UN_IN: u^n is the stage input itself (the first stage, chosen at launch), so its value at the
 // cell is the centre value the combine already receives and is not loaded again (526 us against 590
 // for the two stages of a 128^3 block, 8x4x8 parts).
-template <int TZ, int MODE, bool UN_IN>
+template <int TZ, int MODE, bool UN_IN, class Order = RhsOrder>
 struct TileIODma {
     typedef __attribute__((address_space(3))) double* LdsPtr;
     using Box = PackedBox<TZ>;
@@ -370,7 +390,7 @@ struct TileIODma {
     // wave outside the block stores none.)
     __host__ __device__ static constexpr int younger(int pos) {
         int n = 0;
-        for (int f = pos + 1; f <= pos + NBUF - 2 && f < NV; ++f) n += KW + (UNB && f >= NBUF - 1 ? 1 : 0);
+        for (int f = pos + 1; f <= pos + NBUF - 2 && f < Order::N; ++f) n += KW + (UNB && f >= NBUF - 1 ? 1 : 0);
         return n;
     }
 
@@ -424,8 +444,8 @@ struct TileIODma {
     }
 
     __device__ __forceinline__ void prefetch(int pos) {
-        if (pos >= NV) return;
-        const int v = FIELD_ORDER[pos];
+        if (pos >= Order::N) return;
+        const int v = Order::field(pos);
         const gchar* f = (const gchar*)(in + v * stride);
         // the LDS base is made opaque at every field, so the chunk addresses (M0 values) are
         // recomputed from it with one scalar add each instead of being kept (and spilled) as
@@ -458,7 +478,7 @@ struct TileIODma {
         }
     }
     __device__ __forceinline__ double staged_un(int v) const {
-        return lds[UN0 + (field_pos(v) % NBUF) * UNB + tid];
+        return lds[UN0 + (Order::pos(v) % NBUF) * UNB + tid];
     }
 
     // at most n of this wave's vector memory operations outstanding (n a constant after
@@ -476,7 +496,7 @@ struct TileIODma {
     }
     __device__ const PackedTaps<Box>& strides() const { return taps; }
     __device__ const double* field(int v) {
-        const int pos = field_pos(v);
+        const int pos = Order::pos(v);
         // this wave's loads of field pos have landed and its LDS accesses are done; then the
         // barrier: every wave's loads of pos have landed and every thread is done with field
         // pos - 1, whose buffer the prefetch refills. Written as statements that may touch any
@@ -1289,158 +1309,258 @@ __global__ void dissipation_kernel(BlockDesc b, const double* __restrict__ u, do
 }
 
 // ------------------------------------------------------------------------------------
-// constraint monitor (src/spacetime/ccz4.cpp:941-1159), global-memory stencils
+// constraint monitor (src/spacetime/ccz4.cpp:941-1159)
 // ------------------------------------------------------------------------------------
-struct GlobalCell {
-    const double* u;
-    long stride, c, st[3];
-    double ih[3], ih2[3], ihh[3];
-    __device__ double f(int v, long off) const { return u[v * stride + c + off]; }
-    __device__ double d1(int v, int d) const {
-        const long q = st[d];
-        return ih[d] * (-f(v, 2 * q) + 8.0 * f(v, q) - 8.0 * f(v, -q) + f(v, -2 * q));
-    }
-    __device__ double d2(int v, int a, int b) const {
-        if (a == b) {
-            const long q = st[a];
-            return ih2[a] * (-f(v, 2 * q) + 16.0 * f(v, q) - 30.0 * f(v, 0) + 16.0 * f(v, -q) - f(v, -2 * q));
-        }
-        const long pa = st[a], pb = st[b];
-        const double h = (a == 0) ? ihh[b == 1 ? 0 : 1] : ihh[2];
-        return h * (f(v, pa + pb) - f(v, pa - pb) - f(v, -pa + pb) + f(v, -pa - pb));
-    }
-};
 
-// H at interior cell t of the block and, when mom is not null, M_i into mom[0..2]
-__device__ __forceinline__ double constraint_cell(const BlockDesc& b, const double* __restrict__ u, long t,
-                                                  const Stencil<double>& K, double* mom) {
-    GlobalCell C;
-    C.u = u;
-    C.stride = b.stride;
-    C.c = t;
-    C.st[0] = 1;
-    C.st[1] = b.nt[0];
-    C.st[2] = (long)b.nt[0] * b.nt[1];
+// 4th-order first and (D2) second derivatives of one staged field
+template <bool D2, class ST>
+__device__ __forceinline__ void field_derivs(const double* s, const Stencil<double>& K, const ST& st, double d1[3],
+                                             double dd[6]) {
+    const double c = s[0];
+#pragma unroll
     for (int d = 0; d < 3; ++d) {
-        C.ih[d] = K.ih[d];
-        C.ih2[d] = K.ih2[d];
-        C.ihh[d] = K.ihh[d];
+        const double m1 = st.at(s, d, -1), p1 = st.at(s, d, 1), m2 = st.at(s, d, -2), p2 = st.at(s, d, 2);
+        d1[d] = K.ih[d] * (-p2 + 8.0 * p1 - 8.0 * m1 + m2);
+        if (D2) dd[sym(d, d)] = K.ih2[d] * (-p2 + 16.0 * p1 - 30.0 * c + 16.0 * m1 - m2);
+        pin(d1[d]);
     }
-    const double chi = C.f(CHI, 0);
-    const double Ktr = C.f(KTR, 0);
+    if (D2) {
+        const long x = st.q(0), y = st.q(1), z = st.q(2);
+        dd[1] = K.ihh[0] * (s[x + y] - s[x - y] - s[-x + y] + s[-x - y]);
+        dd[2] = K.ihh[1] * (s[x + z] - s[x - z] - s[-x + z] + s[-x - z]);
+        dd[4] = K.ihh[2] * (s[y + z] - s[y - z] - s[-y + z] + s[-y - z]);
+#pragma unroll
+        for (int q = 0; q < 6; ++q) pin(dd[q]);
+    }
+}
+
+// H of one cell and, with MOM, M_i into mom[0..2]; the fields come staged one by one, each folded
+// into the Ricci tensor (or M_i) as it arrives
+template <bool MOM, class Stager>
+__device__ __forceinline__ double constraint_cell(Stager& S, const Stencil<double>& K, double mom[3]) {
+    const double chi = S.centre(CHI), Ktr = S.centre(KTR);
     double gt[6], At[6], Gh[3];
+#pragma unroll
     for (int a = 0; a < 6; ++a) {
-        gt[a] = C.f(GXX + a, 0);
-        At[a] = C.f(AXX + a, 0);
+        gt[a] = S.centre(GXX + a);
+        At[a] = S.centre(AXX + a);
     }
-    for (int a = 0; a < 3; ++a) Gh[a] = C.f(GHX + a, 0);
+#pragma unroll
+    for (int a = 0; a < 3; ++a) Gh[a] = S.centre(GHX + a);
     const double det = gt[0] * (gt[3] * gt[5] - gt[4] * gt[4]) - gt[1] * (gt[1] * gt[5] - gt[4] * gt[2]) +
         gt[2] * (gt[1] * gt[4] - gt[3] * gt[2]);
     const double idet = 1.0 / (det + 1.0e-30);
     const double gu[6] = {(gt[3] * gt[5] - gt[4] * gt[4]) * idet, (gt[2] * gt[4] - gt[1] * gt[5]) * idet,
                           (gt[1] * gt[4] - gt[2] * gt[3]) * idet, (gt[0] * gt[5] - gt[2] * gt[2]) * idet,
                           (gt[1] * gt[2] - gt[0] * gt[4]) * idet, (gt[0] * gt[3] - gt[1] * gt[1]) * idet};
-    double Au[3][3];
-    for (int a = 0; a < 3; ++a)
-        for (int c = 0; c < 3; ++c)
-            Au[a][c] = gu[sym(a, 0)] * At[sym(0, c)] + gu[sym(a, 1)] * At[sym(1, c)] + gu[sym(a, 2)] * At[sym(2, c)];
     double AA = 0.0;
-    for (int a = 0; a < 3; ++a)
-        for (int c = 0; c < 3; ++c) AA += Au[a][c] * Au[c][a];
-    double dgt[6][3], ddgt[6][6], dchi[3], ddchi[6], dGh[3][3];
-    for (int v = 0; v < 6; ++v)
-        for (int d = 0; d < 3; ++d) {
-            dgt[v][d] = C.d1(GXX + v, d);
-            for (int e = d; e < 3; ++e) ddgt[v][sym(d, e)] = C.d2(GXX + v, d, e);
-        }
-    for (int d = 0; d < 3; ++d) {
-        dchi[d] = C.d1(CHI, d);
-        for (int e = d; e < 3; ++e) ddchi[sym(d, e)] = C.d2(CHI, d, e);
-        for (int a = 0; a < 3; ++a) dGh[a][d] = C.d1(GHX + a, d);
+    {
+        double Au[3][3];
+#pragma unroll
+        for (int a = 0; a < 3; ++a)
+#pragma unroll
+            for (int c = 0; c < 3; ++c)
+                Au[a][c] = gu[sym(a, 0)] * At[sym(0, c)] + gu[sym(a, 1)] * At[sym(1, c)] + gu[sym(a, 2)] * At[sym(2, c)];
+#pragma unroll
+        for (int a = 0; a < 3; ++a)
+#pragma unroll
+            for (int c = 0; c < 3; ++c) AA += Au[a][c] * Au[c][a];
+        pin(AA);
+    }
+
+    // metric: Ricci term -1/2 g^lm d_l d_m gt_ij, first derivatives kept for the Christoffels
+    double dgt[6][3], dd[6], Rt[6];
+#pragma unroll
+    for (int p = 0; p < 6; ++p) {
+        field_derivs<true>(S.field(GXX + p), K, S.strides(), dgt[p], dd);
+        double r = 0.0;
+#pragma unroll
+        for (int q = 0; q < 6; ++q) r += ((q == 0 || q == 3 || q == 5) ? -0.5 : -1.0) * gu[q] * dd[q];
+        Rt[p] = r;
+        pin(Rt[p]);
     }
     double chr[3][6];
+#pragma unroll
     for (int q = 0; q < 3; ++q)
+#pragma unroll
         for (int p = 0; p < 6; ++p) {
             const int a = sym_a(p), c = sym_b(p);
-            double s = 0.0;
-            for (int m = 0; m < 3; ++m) s += gu[sym(q, m)] * (dgt[sym(m, a)][c] + dgt[sym(m, c)][a] - dgt[p][m]);
-            chr[q][p] = 0.5 * s;
+            double v = 0.0;
+#pragma unroll
+            for (int m = 0; m < 3; ++m) v += gu[sym(q, m)] * (dgt[sym(m, a)][c] + dgt[sym(m, c)][a] - dgt[p][m]);
+            chr[q][p] = 0.5 * v;
+            pin(chr[q][p]);
         }
-    double G[3][6];
-    for (int q = 0; q < 3; ++q)
-        for (int p = 0; p < 6; ++p) G[q][p] = gt[sym(q, 0)] * chr[0][p] + gt[sym(q, 1)] * chr[1][p] + gt[sym(q, 2)] * chr[2][p];
-    double Gd[3];
-    for (int q = 0; q < 3; ++q) {
-        double s = 0.0;
-        for (int p = 0; p < 6; ++p) s += ((p == 0 || p == 3 || p == 5) ? 1.0 : 2.0) * gu[p] * chr[q][p];
-        Gd[q] = s;
+
+    // chi: the conformal-factor part of the Ricci tensor
+    double dchi[3];
+    field_derivs<true>(S.field(CHI), K, S.strides(), dchi, dd);
+    {
+        double D[6], lapchi = 0.0, gradchi2 = 0.0;
+#pragma unroll
+        for (int p = 0; p < 6; ++p) {
+            const int l = sym_a(p), m = sym_b(p);
+            const double f = (l == m) ? 1.0 : 2.0;
+            D[p] = dd[p] - chr[0][p] * dchi[0] - chr[1][p] * dchi[1] - chr[2][p] * dchi[2];
+            lapchi += f * gu[p] * D[p];
+            gradchi2 += f * gu[p] * dchi[l] * dchi[m];
+        }
+#pragma unroll
+        for (int p = 0; p < 6; ++p)
+            Rt[p] += (0.5 / (chi + 1e-30)) * (D[p] + gt[p] * lapchi) -
+                (0.25 / ((chi * chi) + 1e-30)) * (dchi[sym_a(p)] * dchi[sym_b(p)] - 3.0 * gt[p] * gradchi2);
     }
-    double lapchi = 0.0, gradchi2 = 0.0;
-    for (int p = 0; p < 6; ++p) {
-        const int l = sym_a(p), m = sym_b(p);
-        const double f = (l == m) ? 1.0 : 2.0;
-        lapchi += f * gu[p] * (ddchi[p] - chr[0][p] * dchi[0] - chr[1][p] * dchi[1] - chr[2][p] * dchi[2]);
-        gradchi2 += f * gu[p] * dchi[l] * dchi[m];
+
+    // products of Christoffel symbols, factored per k as in ccz4_cell
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        double Gk[6], Gd = 0.0;
+#pragma unroll
+        for (int p = 0; p < 6; ++p) {
+            Gk[p] = gt[sym(k, 0)] * chr[0][p] + gt[sym(k, 1)] * chr[1][p] + gt[sym(k, 2)] * chr[2][p];
+            Gd += ((p == 0 || p == 3 || p == 5) ? 1.0 : 2.0) * gu[p] * chr[k][p];
+        }
+#pragma unroll
+        for (int p = 0; p < 6; ++p) Rt[p] += (Gh[k] - Gd) * Gk[p];
+#pragma unroll
+        for (int l = 0; l < 3; ++l) {
+            double H[3];
+#pragma unroll
+            for (int j = 0; j < 3; ++j)
+                H[j] = gu[sym(l, 0)] * Gk[sym(j, 0)] + gu[sym(l, 1)] * Gk[sym(j, 1)] + gu[sym(l, 2)] * Gk[sym(j, 2)];
+#pragma unroll
+            for (int p = 0; p < 6; ++p) {
+                const int a = sym_a(p), b = sym_b(p);
+                Rt[p] += chr[k][sym(l, a)] * H[b] + chr[k][sym(l, b)] * H[a];
+            }
+        }
+    }
+#pragma unroll
+    for (int p = 0; p < 6; ++p) pin(Rt[p]);
+
+    double d1[3];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+        field_derivs<false>(S.field(GHX + q), K, S.strides(), d1, dd);
+#pragma unroll
+        for (int p = 0; p < 6; ++p) {
+            const int a = sym_a(p), b = sym_b(p);
+            Rt[p] += 0.5 * (gt[sym(q, a)] * d1[b] + gt[sym(q, b)] * d1[a]);
+            pin(Rt[p]);
+        }
     }
     double Rs = 0.0;
-    for (int p = 0; p < 6; ++p) {
-        const int a = sym_a(p), c = sym_b(p);
-        double R = 0.0;
-        for (int q = 0; q < 6; ++q) R += ((q == 0 || q == 3 || q == 5) ? -0.5 : -1.0) * gu[q] * ddgt[p][q];
-        for (int q = 0; q < 3; ++q) {
-            R += 0.5 * (gt[sym(q, a)] * dGh[q][c] + gt[sym(q, c)] * dGh[q][a]);
-            R += (Gh[q] - Gd[q]) * G[q][p];
-            for (int l = 0; l < 3; ++l) {
-                const double Hc = gu[sym(l, 0)] * G[q][sym(c, 0)] + gu[sym(l, 1)] * G[q][sym(c, 1)] + gu[sym(l, 2)] * G[q][sym(c, 2)];
-                const double Ha = gu[sym(l, 0)] * G[q][sym(a, 0)] + gu[sym(l, 1)] * G[q][sym(a, 1)] + gu[sym(l, 2)] * G[q][sym(a, 2)];
-                R += chr[q][sym(l, a)] * Hc + chr[q][sym(l, c)] * Ha;
-            }
-        }
-        const double Dab = ddchi[p] - chr[0][p] * dchi[0] - chr[1][p] * dchi[1] - chr[2][p] * dchi[2];
-        const double Rc = (0.5 / (chi + 1e-30)) * (Dab + gt[p] * lapchi) -
-            (0.25 / ((chi * chi) + 1e-30)) * (dchi[a] * dchi[c] - 3.0 * gt[p] * gradchi2);
-        Rs += ((p == 0 || p == 3 || p == 5) ? 1.0 : 2.0) * gu[p] * (R + Rc);
-    }
+#pragma unroll
+    for (int p = 0; p < 6; ++p) Rs += ((p == 0 || p == 3 || p == 5) ? 1.0 : 2.0) * gu[p] * Rt[p];
     Rs *= chi;
-    const double H = Rs + (2.0 / 3.0) * Ktr * Ktr - AA;
-    if (!mom) return H;
-    double dAt[6][3], dK[3];
-    for (int v = 0; v < 6; ++v)
-        for (int d = 0; d < 3; ++d) dAt[v][d] = C.d1(AXX + v, d);
-    for (int d = 0; d < 3; ++d) dK[d] = C.d1(KTR, d);
+    double H = Rs + (2.0 / 3.0) * Ktr * Ktr - AA;
+    pin(H);
+    if (!MOM) return H;
+
+    // M_a = g^cq (d_c A_qa - chr^m_cq A_ma - chr^m_ca A_qm - 3 / (2 chi) A_ac d_q chi) - 2/3 d_a K:
+    // the terms of the cell itself, then K's and A~'s derivatives as the fields arrive
+    const double c3 = 3.0 / (2.0 * chi + 1e-30);
+#pragma unroll
     for (int a = 0; a < 3; ++a) {
         double M = 0.0;
+#pragma unroll
         for (int c = 0; c < 3; ++c)
+#pragma unroll
             for (int q = 0; q < 3; ++q) {
-                const double gcq = gu[sym(c, q)];
-                double DA = dAt[sym(q, a)][c];
+                double DA = -c3 * At[sym(a, c)] * dchi[q];
+#pragma unroll
                 for (int m = 0; m < 3; ++m) DA -= chr[m][sym(c, q)] * At[sym(m, a)] + chr[m][sym(c, a)] * At[sym(q, m)];
-                M += gcq * DA;
-                M -= (3.0 / (2.0 * chi + 1e-30)) * At[sym(a, c)] * gcq * dchi[q];
+                M += gu[sym(c, q)] * DA;
             }
-        M -= (2.0 / 3.0) * dK[a];
         mom[a] = M;
+        pin(mom[a]);
+    }
+    field_derivs<false>(S.field(KTR), K, S.strides(), d1, dd);
+#pragma unroll
+    for (int a = 0; a < 3; ++a) mom[a] -= (2.0 / 3.0) * d1[a];
+#pragma unroll
+    for (int p = 0; p < 6; ++p) {
+        const int i = sym_a(p), j = sym_b(p);
+        field_derivs<false>(S.field(AXX + p), K, S.strides(), d1, dd);
+        mom[j] += gu[sym(0, i)] * d1[0] + gu[sym(1, i)] * d1[1] + gu[sym(2, i)] * d1[2];
+        if (i != j) mom[i] += gu[sym(0, j)] * d1[0] + gu[sym(1, j)] * d1[1] + gu[sym(2, j)] * d1[2];
+#pragma unroll
+        for (int a = 0; a < 3; ++a) pin(mom[a]);
     }
     return H;
 }
 
-__global__ void constraints_kernel(BlockDesc b, const double* __restrict__ u, double* ham, double* mom,
-                                   Stencil<double> K) {
-    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= b.stride) return;
-    const int i = (int)(t % b.nt[0]);
-    const int j = (int)((t / b.nt[0]) % b.nt[1]);
-    const int k = (int)(t / ((long)b.nt[0] * b.nt[1]));
-    const bool inner = i >= b.ng && i < b.ng + b.n[0] && j >= b.ng && j < b.ng + b.n[1] && k >= b.ng &&
-        k < b.ng + b.n[2];
-    if (!inner) {
-        ham[t] = 0.0;
-        if (mom) mom[3 * t] = mom[3 * t + 1] = mom[3 * t + 2] = 0.0;
-        return;
+__device__ __forceinline__ double part_sum(double v, double* sh, int n) {
+    sh[threadIdx.x] = v;
+    __syncthreads();
+    for (int o = n / 2; o > 0; o >>= 1) {
+        if ((int)threadIdx.x < o) sh[threadIdx.x] += sh[threadIdx.x + o];
+        __syncthreads();
     }
-    ham[t] = constraint_cell(b, u, t, K, mom ? mom + 3 * t : nullptr);
+    const double s = sh[0];
+    __syncthreads();
+    return s;
 }
 
+// H (and, with MOM, M_i) over one block, in the stage kernel's parts and staging: each workgroup
+// takes `per` consecutive parts. ham / mom (may be null): the values per interior cell, mom cell-major;
+// partial (may be null): per workgroup the sum of H^2 and, gridDim.x further on, of |M|^2. 183 us for H
+// and M_i of 10^6 cells (132x96x96, 17 fields of the state at 0.8 TB/s: bound as the stage kernel is,
+// by the cache lines of the halo and the arithmetic); with the stencils read from memory by every
+// cell and 1.9 KB of scratch per lane it took 1463 us.
+template <bool MOM>
+__global__ __launch_bounds__(64 * TZ_LARGE, 2) void constraints_kernel(StageArgs A, double* ham, double* mom,
+                                                                       double* partial, int per) {
+    constexpr int TZ = TZ_LARGE, NT = 64 * TZ;
+    using IO = TileIODma<TZ, MODE_RHS, false, MonitorOrder<MOM>>;
+    __shared__ __align__(16) double lds[IO::LDS_DOUBLES];
+    const int tid = threadIdx.x;
+    const int nparts = A.ntiles * FP64_PARTS<TZ>;
+    const int first = tile_of_block(blockIdx.x, gridDim.x, A.xcd_remap) * per;
+    const int last = first + per < nparts ? first + per : nparts;
+    int lx = 0, ly = 0, lz = 0;
+    LaneMap<TZ>::cell(tid, lx, ly, lz);
+    double h2 = 0.0, m2 = 0.0;
+    for (int part = first; part < last; ++part) {
+        const TileRef R = resolve_tile(A, part / FP64_PARTS<TZ>);
+        const BlockDesc& b = R.b;
+        const int x0 = R.tix * TILE_X, y0 = R.tiy * TILE_Y, z0 = R.tiz * TILE_Z + part % FP64_PARTS<TZ> * TZ;
+        if (z0 >= b.n[2]) continue; // uniform over the workgroup
+        const int ix = x0 + lx, iy = y0 + ly, iz = z0 + lz;
+        const bool active = ix < b.n[0] && iy < b.n[1] && iz < b.n[2];
+        const int gi = b.ng + (active ? ix : 0), gj = b.ng + (active ? iy : 0), gk = b.ng + (active ? iz : 0);
+        const long cidx = gi + (long)b.nt[0] * (gj + (long)b.nt[1] * gk);
+        IO io;
+        io.lds = lds;
+        io.in = R.in;
+        io.stride = b.stride;
+        io.cb = 8u * (unsigned)cidx;
+        io.place(lx, ly, lz);
+        io.init(tid, b.ng + x0, b.ng + y0, b.ng + z0, b);
+        double M[3] = {0.0, 0.0, 0.0};
+        const double H = constraint_cell<MOM>(io, A.K, M);
+        if (active) {
+            h2 += H * H;
+            if (MOM) m2 += M[0] * M[0] + M[1] * M[1] + M[2] * M[2];
+            if (ham) ham[cidx] = H;
+            if (MOM && mom)
+#pragma unroll
+                for (int a = 0; a < 3; ++a) mom[3 * cidx + a] = M[a];
+        }
+        __syncthreads(); // the next part reuses the buffers
+    }
+    if (!partial) return;
+    const double sh2 = part_sum(h2, lds, NT);
+    const double sm2 = MOM ? part_sum(m2, lds, NT) : 0.0;
+    if (tid == 0) {
+        partial[blockIdx.x] = sh2;
+        if (MOM) partial[gridDim.x + blockIdx.x] = sm2;
+    }
+}
+
+__global__ void zero_kernel(double* p, long n) {
+    for (long t = (long)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (long)gridDim.x * blockDim.x) p[t] = 0.0;
+}
 
 // ------------------------------------------------------------------------------------
 // initial data and noise
@@ -1519,50 +1639,6 @@ __device__ __forceinline__ double block_sum(double v, double* sh) {
     return sh[0];
 }
 
-// sum over the interior cells of the squares of an array of ncomp values per cell
-// (cell-major, as the reference's ham and mom arrays)
-__global__ __launch_bounds__(RED_T) void sumsq_kernel(BlockDesc b, const double* ham, int ncomp, double* partial,
-                                                      long per) {
-    __shared__ double sh[RED_T];
-    const long ncell = (long)b.n[0] * b.n[1] * b.n[2];
-    const long beg = (long)blockIdx.x * per;
-    const long end = beg + per < ncell ? beg + per : ncell;
-    double acc = 0.0;
-    for (long t = beg + threadIdx.x; t < end; t += RED_T) {
-        const int i = b.ng + (int)(t % b.n[0]);
-        const int j = b.ng + (int)((t / b.n[0]) % b.n[1]);
-        const int k = b.ng + (int)(t / ((long)b.n[0] * b.n[1]));
-        const long c = i + (long)b.nt[0] * (j + (long)b.nt[1] * k);
-        for (int a = 0; a < ncomp; ++a) {
-            const double h = ham[ncomp * c + a];
-            acc += h * h;
-        }
-    }
-    const double s = block_sum(acc, sh);
-    if (threadIdx.x == 0) partial[blockIdx.x] = s;
-}
-
-// sum over the interior of H^2 with H formed on the fly (no per-cell H array): the partition
-// and the visiting order of sumsq_kernel over constraints_kernel's output
-__global__ __launch_bounds__(RED_T) void ham_sumsq_kernel(BlockDesc b, const double* __restrict__ u,
-                                                          Stencil<double> K, double* partial, long per) {
-    __shared__ double sh[RED_T];
-    const long ncell = (long)b.n[0] * b.n[1] * b.n[2];
-    const long beg = (long)blockIdx.x * per;
-    const long end = beg + per < ncell ? beg + per : ncell;
-    double acc = 0.0;
-    for (long t = beg + threadIdx.x; t < end; t += RED_T) {
-        const int i = b.ng + (int)(t % b.n[0]);
-        const int j = b.ng + (int)((t / b.n[0]) % b.n[1]);
-        const int k = b.ng + (int)(t / ((long)b.n[0] * b.n[1]));
-        const long c = i + (long)b.nt[0] * (j + (long)b.nt[1] * k);
-        const double h = constraint_cell(b, u, c, K, nullptr);
-        acc += h * h;
-    }
-    const double s = block_sum(acc, sh);
-    if (threadIdx.x == 0) partial[blockIdx.x] = s;
-}
-
 __global__ __launch_bounds__(RED_T) void nonfinite_kernel(BlockDesc b, const double* u, double* partial, long per) {
     __shared__ double sh[RED_T];
     const long ncell = (long)b.n[0] * b.n[1] * b.n[2];
@@ -1580,12 +1656,13 @@ __global__ __launch_bounds__(RED_T) void nonfinite_kernel(BlockDesc b, const dou
     if (threadIdx.x == 0) partial[blockIdx.x] = s;
 }
 
+// out[g] = sum of the n partials of group g (one workgroup per group)
 __global__ __launch_bounds__(RED_T) void sum_partials_kernel(const double* partial, int n, double* out) {
     __shared__ double sh[RED_T];
     double acc = 0.0;
-    for (int t = threadIdx.x; t < n; t += RED_T) acc += partial[t];
+    for (int t = threadIdx.x; t < n; t += RED_T) acc += partial[(long)blockIdx.x * n + t];
     const double s = block_sum(acc, sh);
-    if (threadIdx.x == 0) out[0] = s;
+    if (threadIdx.x == 0) out[blockIdx.x] = s;
 }
 
 // First non-finite interior value in the order of the reference's NaN scan
@@ -1956,9 +2033,43 @@ hipError_t launch_dissipation(const BlockDesc& b, const double* u, double* rhs, 
     return hipGetLastError();
 }
 
+// workgroups and parts per workgroup of a monitor launch with at most `cap` workgroups; sums take
+// the 512 that run together (two per CU), so that each has the same number of parts but one
+constexpr int MONITOR_GROUPS = 512;
+static int monitor_split(int ntiles, int cap, int* per) {
+    const int nparts = ntiles * FP64_PARTS<TZ_LARGE>;
+    *per = (nparts + cap - 1) / cap;
+    return (nparts + *per - 1) / *per;
+}
+
+static hipError_t launch_monitor(const BlockDesc& b, const double* u, double* ham, double* mom, bool with_mom,
+                                 double* partial, int cap, int* groups, hipStream_t s) {
+    static const int sel[3] = {0, 0, 0};
+    const StageArgs A = stage_args(single_batch(b, u, u, nullptr), sel, CellParams{}, 0.0, StageCoef{0.0, 0.0, 0.0},
+                                   nullptr, 0);
+    int per = 1;
+    *groups = monitor_split(A.ntiles, cap, &per);
+    if (with_mom)
+        constraints_kernel<true><<<*groups, 64 * TZ_LARGE, 0, s>>>(A, ham, mom, partial, per);
+    else
+        constraints_kernel<false><<<*groups, 64 * TZ_LARGE, 0, s>>>(A, ham, nullptr, partial, per);
+    return hipGetLastError();
+}
+
 hipError_t launch_constraints(const BlockDesc& b, const double* u, double* ham, double* mom, hipStream_t s) {
-    constraints_kernel<<<grid_for(b.stride, 128), 128, 0, s>>>(b, u, ham, mom,
-                                                              make_stencil(b, 0.0));
+    zero_kernel<<<grid_for(b.stride, 256 * 4), 256, 0, s>>>(ham, b.stride);
+    if (mom) zero_kernel<<<grid_for(3 * b.stride, 256 * 4), 256, 0, s>>>(mom, 3 * b.stride);
+    int groups = 0;
+    return launch_monitor(b, u, ham, mom, mom != nullptr, nullptr, 1 << 30, &groups, s);
+}
+
+hipError_t launch_constraint_sums(const BlockDesc& b, const double* u, bool with_mom, double* partial, int cap,
+                                  double* out, hipStream_t s) {
+    int groups = 0;
+    const hipError_t st = launch_monitor(b, u, nullptr, nullptr, with_mom, partial,
+                                         cap < MONITOR_GROUPS ? cap : MONITOR_GROUPS, &groups, s);
+    if (st != hipSuccess) return st;
+    sum_partials_kernel<<<with_mom ? 2 : 1, RED_T, 0, s>>>(partial, groups, out);
     return hipGetLastError();
 }
 
@@ -1980,26 +2091,6 @@ static long reduce_split(const BlockDesc& b, int cap, int* nparts) {
     if (per < RED_T) per = RED_T;
     *nparts = (int)((ncell + per - 1) / per);
     return per;
-}
-
-hipError_t launch_sumsq_interior(const BlockDesc& b, const double* ham, int ncomp, double* partial, int cap,
-                                 int* nparts, hipStream_t s) {
-    const long per = reduce_split(b, cap, nparts);
-    sumsq_kernel<<<*nparts, RED_T, 0, s>>>(b, ham, ncomp, partial, per);
-    return hipGetLastError();
-}
-
-int reduce_parts(const BlockDesc& b, int cap) {
-    int n = 0;
-    (void)reduce_split(b, cap, &n);
-    return n;
-}
-
-hipError_t launch_ham_sumsq(const BlockDesc& b, const double* u, double* partial, int cap, int* nparts,
-                            hipStream_t s) {
-    const long per = reduce_split(b, cap, nparts);
-    ham_sumsq_kernel<<<*nparts, RED_T, 0, s>>>(b, u, make_stencil(b, 0.0), partial, per);
-    return hipGetLastError();
 }
 
 hipError_t launch_count_nonfinite(const BlockDesc& b, const double* u, double* partial, int cap, int* nparts,

@@ -152,18 +152,12 @@ hipError_t launch_init_bl(const BlockDesc& b, double* u, int nbh, const double* 
 hipError_t launch_add_noise(const BlockDesc& b, double* u, unsigned long long seed, double amp, unsigned mask,
                             hipStream_t s);
 
-// partial[blockIdx] = sum over interior cells of the squares of the ncomp values per cell
-// (ncomp 1: ham, 3: mom); count is analytic. Returns the number of partials written in
-// *nparts (<= cap).
-hipError_t launch_sumsq_interior(const BlockDesc& b, const double* ham, int ncomp, double* partial, int cap,
-                                 int* nparts, hipStream_t s);
+// out[0] = sum of H^2 over the interior and, with_mom, out[1] = sum of |M|^2. partial: scratch of cap
+// doubles (2 * cap with_mom).
+hipError_t launch_constraint_sums(const BlockDesc& b, const double* u, bool with_mom, double* partial, int cap,
+                                  double* out, hipStream_t s);
 // sums `n` doubles into out[0] with one workgroup (fixed order)
 hipError_t launch_sum_partials(const double* partial, int n, double* out, hipStream_t s);
-// number of partials the interior reductions split a block into (at most `cap`)
-int reduce_parts(const BlockDesc& b, int cap);
-// partial sums of H^2 over the interior (H formed on the fly), at most `cap` partials
-hipError_t launch_ham_sumsq(const BlockDesc& b, const double* u, double* partial, int cap, int* nparts,
-                            hipStream_t s);
 // partial[blockIdx] = number of non-finite interior values over all 22 fields
 hipError_t launch_count_nonfinite(const BlockDesc& b, const double* u, double* partial, int cap, int* nparts,
                                   hipStream_t s);
