@@ -83,16 +83,24 @@ template <int SX, int SY, int SZ>
 struct FixedStrides {
     static constexpr bool READS_FIRST = false;
     __host__ __device__ static constexpr long q(int d) { return d == 0 ? SX : (d == 1 ? SY : SZ); }
-    // value k cells off along axis d
+    // value at the cell, k cells off along axis d, and i cells off along a and j along b
+    template <typename R>
+    __host__ __device__ static R centre(const R* s) { return s[0]; }
     template <typename R>
     __host__ __device__ static R at(const R* s, int d, int k) { return s[k * q(d)]; }
+    template <typename R>
+    __host__ __device__ static R edge(const R* s, int a, int b, int i, int j) { return s[i * q(a) + j * q(b)]; }
 };
 struct RuntimeStrides {
     static constexpr bool READS_FIRST = false;
     long s[3];
     __host__ __device__ long q(int d) const { return s[d]; }
     template <typename R>
+    __host__ __device__ static R centre(const R* p) { return p[0]; }
+    template <typename R>
     __host__ __device__ R at(const R* p, int d, int k) const { return p[k * s[d]]; }
+    template <typename R>
+    __host__ __device__ R edge(const R* p, int a, int b, int i, int j) const { return p[i * s[a] + j * s[b]]; }
 };
 
 struct CellParams {
@@ -198,7 +206,7 @@ struct Advection {
 template <bool D2, bool KO_EXACT, typename R, class ST>
 __host__ __device__ GR_INLINE void eval_field(const R* s, const Stencil<R>& K, const ST& st, const Advection<R>& B,
                                               R d1[3], R dd[6], R& adv, R& ko) {
-    const R c = s[0];
+    const R c = st.centre(s);
     R upS = R(0), cenS = R(0);
     adv = R(0);
 #pragma unroll
@@ -224,10 +232,12 @@ __host__ __device__ GR_INLINE void eval_field(const R* s, const Stencil<R>& K, c
         if (D2) dd[sym(d, d)] = K.ih2[d] * (-p2 + R(16) * p1 - R(30) * c + R(16) * m1 - m2);
     }
     if (D2) {
-        const long x = st.q(0), y = st.q(1), z = st.q(2);
-        dd[1] = K.ihh[0] * (s[x + y] - s[x - y] - s[-x + y] + s[-x - y]);
-        dd[2] = K.ihh[1] * (s[x + z] - s[x - z] - s[-x + z] + s[-x - z]);
-        dd[4] = K.ihh[2] * (s[y + z] - s[y - z] - s[-y + z] + s[-y - z]);
+        auto mixed = [&](int a, int b) {
+            return st.edge(s, a, b, 1, 1) - st.edge(s, a, b, 1, -1) - st.edge(s, a, b, -1, 1) + st.edge(s, a, b, -1, -1);
+        };
+        dd[1] = K.ihh[0] * mixed(0, 1);
+        dd[2] = K.ihh[1] * mixed(0, 2);
+        dd[4] = K.ihh[2] * mixed(1, 2);
     }
     if (!B.FOLDED) adv = B.w * upS + (R(1) - B.w) * cenS;
 #ifdef __HIP_DEVICE_COMPILE__

@@ -304,22 +304,47 @@ struct PackedBox {
         return true;
     }
 };
-// Taps of a packed box: the z taps two cells off and more have an address of their own per lane.
+// Taps of a packed box. The z taps two cells off and more have an address of their own per lane; the
+// others are reached from three bases per buffer, below the taps of the cell's own plane and of
+// the planes next to it, each near enough for the paired LDS reads' 8-bit offsets: from the cell
+// itself the compiler adds an address for nearly every pair, 228 instructions a part (128^3,
+// stages 1-2: 504 -> 497 us; the uneven 64 blocks 772 -> 762).
 template <class Box>
 struct PackedTaps {
+    typedef const __attribute__((address_space(3))) double* LdsPtr;
+    static constexpr int NB = 4; // buffers, at most
+    LdsPtr z[6];        // z - 4, - 3, - 2, + 2, + 3, + 4 in buffer 0
+    LdsPtr base[NB][3]; // per buffer: planes z - 1, z, z + 1
+    int buf, ofs;       // the current field's buffer and its first double
     // the small parts run one wave per SIMD, with no other to cover a wait: all LDS reads of a field
     // ahead of its arithmetic (a 16^3 stage 23.4 -> 21.3 us, 32^3 25.3 -> 23.4). With two waves
     // the registers that costs are worth more (128^3: 519 us against 508 without).
     static constexpr bool READS_FIRST = Box::NP == 2 + 2 * HALO;
-    typedef const __attribute__((address_space(3))) double* LdsPtr;
-    LdsPtr z[6]; // z - 4, - 3, - 2, + 2, + 3, + 4 in buffer 0
-    int ofs;     // first double of the current field's buffer
-    __device__ static constexpr long q(int d) {
-        return d == 0 ? 1 : (d == 1 ? Box::ROW : Box::PL);
+    __device__ static constexpr int low(int p) { return p == 1 ? -HALO * Box::ROW : (p - 1) * Box::PL - Box::ROW; }
+    __device__ __forceinline__ void place(LdsPtr lds, int lx, int ly, int lz, int nbuf, int size) {
+#pragma unroll
+        for (int k = 0; k < 6; ++k) z[k] = lds + Box::pos(lx, ly, lz + (k < 3 ? k - 4 : k - 1));
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int p = 0; p < 3; ++p) {
+                if (b >= nbuf) continue;
+                base[b][p] = lds + Box::pos(lx, ly, lz) + b * size + low(p);
+#ifdef __HIP_DEVICE_COMPILE__
+                asm("" : "+v"(base[b][p])); // kept as one address: offsets from it fit the reads
+#endif
+            }
     }
-    __device__ __forceinline__ double at(const double* s, int d, int k) const {
+    __device__ __forceinline__ double near(int dz, int q) const { return base[buf][dz + 1][q - low(dz + 1) + dz * Box::PL]; }
+    __device__ __forceinline__ double at(const double*, int d, int k) const {
         if (d == 2 && (k >= 2 || k <= -2)) return z[k < 0 ? k + 4 : k + 1][ofs];
-        return s[k * q(d)];
+        return d == 2 ? near(k, 0) : near(0, d == 1 ? k * Box::ROW : k);
+    }
+    __device__ __forceinline__ double centre(const double*) const { return near(0, 0); }
+    // i cells along axis a and j along axis b > a (i, j = -1 or 1)
+    __device__ __forceinline__ double edge(const double*, int a, int b, int i, int j) const {
+        const int q = a == 0 ? i : i * Box::ROW;
+        return b == 2 ? near(j, q) : near(0, q + j * Box::ROW);
     }
 };
 
@@ -382,7 +407,9 @@ struct TileIODma {
     static constexpr int fits(int n) { return (n * (LBUF + UNB) + METRIC) * 8 * 2 <= 163840; }
     static constexpr int NBUF = fits(4) ? 4 : 3;
     static_assert(fits(NBUF), "field buffers");
-    static constexpr int UN0 = NBUF * LBUF, METRIC0 = UN0 + NBUF * UNB; // first double of each region
+    // first double of each region (u^n first, so that every LDS address is a lane's own plus an
+    // immediate offset of 16 bits)
+    static constexpr int BUF0 = NBUF * UNB, METRIC0 = BUF0 + NBUF * LBUF;
     static constexpr int LDS_DOUBLES = METRIC0 + METRIC;
     // vector memory operations a wave issues after its loads of field `pos` and before the
     // barrier of that field, at least: in each turn between, the loads of one more field with its
@@ -400,7 +427,6 @@ struct TileIODma {
     gdouble* out;
     long stride;
     unsigned cb; // byte offset of the thread's cell inside one field
-    int cl;
     int wave;
     bool active;
     bool ko_on;
@@ -413,9 +439,7 @@ struct TileIODma {
     double hA[6];
 
     __device__ __forceinline__ void place(int lx, int ly, int lz) {
-        cl = Box::pos(lx, ly, lz);
-#pragma unroll
-        for (int k = 0; k < 6; ++k) taps.z[k] = (LdsPtr)lds + Box::pos(lx, ly, lz + (k < 3 ? k - 4 : k - 1));
+        taps.place((LdsPtr)lds + BUF0, lx, ly, lz, NBUF, LBUF);
     }
 
     // byte offset of the pair at (x, y, z) of the part, or of the part's first pair where it lies
@@ -455,8 +479,8 @@ struct TileIODma {
         asm volatile("" : "+s"(base));
 #endif
         LdsPtr L = (LdsPtr)(uintptr_t)base;
-        const LdsPtr U = L + UN0 + (pos % NBUF) * UNB + wave * 64;
-        L += (pos % NBUF) * LBUF;
+        const LdsPtr U = L + (pos % NBUF) * UNB + wave * 64;
+        L += BUF0 + (pos % NBUF) * LBUF;
 #pragma unroll
         for (int k = 0; k < KW; ++k) {
             const int c = wave + k * NW; // uniform over the wave
@@ -478,7 +502,7 @@ struct TileIODma {
         }
     }
     __device__ __forceinline__ double staged_un(int v) const {
-        return lds[UN0 + (Order::pos(v) % NBUF) * UNB + tid];
+        return lds[(Order::pos(v) % NBUF) * UNB + tid];
     }
 
     // at most n of this wave's vector memory operations outstanding (n a constant after
@@ -508,8 +532,9 @@ struct TileIODma {
 #endif
         prefetch(pos + NBUF - 1);
         if (UNB && v >= AXX && v < AXX + 6) unA[v - AXX] = staged_un(v);
+        taps.buf = pos % NBUF;
         taps.ofs = (pos % NBUF) * LBUF;
-        return lds + (pos % NBUF) * LBUF + cl;
+        return lds; // the taps know the cell
     }
 
     // ---- Sink
@@ -1316,7 +1341,7 @@ __global__ void dissipation_kernel(BlockDesc b, const double* __restrict__ u, do
 template <bool D2, class ST>
 __device__ __forceinline__ void field_derivs(const double* s, const Stencil<double>& K, const ST& st, double d1[3],
                                              double dd[6]) {
-    const double c = s[0];
+    const double c = st.centre(s);
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
         const double m1 = st.at(s, d, -1), p1 = st.at(s, d, 1), m2 = st.at(s, d, -2), p2 = st.at(s, d, 2);
@@ -1325,10 +1350,12 @@ __device__ __forceinline__ void field_derivs(const double* s, const Stencil<doub
         pin(d1[d]);
     }
     if (D2) {
-        const long x = st.q(0), y = st.q(1), z = st.q(2);
-        dd[1] = K.ihh[0] * (s[x + y] - s[x - y] - s[-x + y] + s[-x - y]);
-        dd[2] = K.ihh[1] * (s[x + z] - s[x - z] - s[-x + z] + s[-x - z]);
-        dd[4] = K.ihh[2] * (s[y + z] - s[y - z] - s[-y + z] + s[-y - z]);
+        auto mixed = [&](int a, int b) {
+            return st.edge(s, a, b, 1, 1) - st.edge(s, a, b, 1, -1) - st.edge(s, a, b, -1, 1) + st.edge(s, a, b, -1, -1);
+        };
+        dd[1] = K.ihh[0] * mixed(0, 1);
+        dd[2] = K.ihh[1] * mixed(0, 2);
+        dd[4] = K.ihh[2] * mixed(1, 2);
 #pragma unroll
         for (int q = 0; q < 6; ++q) pin(dd[q]);
     }
