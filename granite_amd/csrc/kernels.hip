@@ -1015,6 +1015,14 @@ __device__ __forceinline__ double f_inf(int v) {
     return (v == 0 || v == 1 || v == 4 || v == 6 || v == 18) ? 1.0 : 0.0;
 }
 
+// a / b from inv = 1 / b, correctly rounded: the quotient, its exact remainder and one correction
+// (Markstein's theorem), with the hardware's rule for zeros, infinities and NaN. Four instructions
+// where a division by itself takes eleven.
+__device__ __forceinline__ double quotient(double a, double b, double inv) {
+    const double q = a * inv;
+    return __builtin_amdgcn_div_fixup(fma(fma(-q, b, a), inv, q), b, a);
+}
+
 // Final value of a ghost cell after the reference's three passes: each pass over axis d
 // rewrites the ghost layers of d over the full transverse extent from the boundary layer,
 // so a cell that is a ghost along a set of axes ends with the chain of 1/r fall-offs from
@@ -1031,6 +1039,10 @@ __device__ __forceinline__ long ghost_count(const BlockDesc& b) {
 // (src/amr/amr.cpp:412-480).
 // Fields g, g + G, ... of the cell: the G field groups run as separate workgroups (second
 // grid dimension), so a small ghost region still fills the machine.
+// Bound by memory: at 192^3 91 us for 145 MB read and 159 MB written, 56 us of them (6 of these the
+// launch's) the x columns, which read two 64-byte lines and write one per row end and field. With
+// the division by a shared reciprocal and each such line written by neighbouring lanes at once:
+// 192^3 95 -> 91 us, 128^3 42.4 -> 40.7, the 64 uneven blocks (four launches) 206 -> 199.
 template <int G>
 __device__ void fill_ghost_cell(const BlockDesc& b, gdouble* u, long t_, int mode, int faces, int g) {
 #pragma clang fp contract(off)
@@ -1055,12 +1067,16 @@ __device__ void fill_ghost_cell(const BlockDesc& b, gdouble* u, long t_, int mod
         k = ng + r / g2;
         j = jj < ng ? jj : b.n[1] + jj;
     } else {
+        // 2 * ng threads per row: the high ghosts of the row before (of the plane's last row at its
+        // first) and the low ghosts of this one, which are neighbours in memory
         const int q = t - nA - nB;
         const int ii = q % g2;
         const int r = q / g2;
-        j = ng + r % b.n[1];
+        const int row = r % b.n[1];
         k = ng + r / b.n[1];
-        i = ii < ng ? ii : b.n[0] + ii;
+        const bool hi = ii < ng;
+        i = hi ? b.nt[0] - ng + ii : ii - ng;
+        j = ng + (hi ? (row > 0 ? row : b.n[1]) - 1 : row);
     }
     const int I[3] = {i, j, k};
     int A[3];
@@ -1098,10 +1114,11 @@ __device__ void fill_ghost_cell(const BlockDesc& b, gdouble* u, long t_, int mod
             const double rin = radius(Q[0], Q[1], Q[2]);
             Q[d] = coord(b, d, I[d]);
             const double rgh = radius(Q[0], Q[1], Q[2]);
+            const double inv = 1.0 / rgh;
 #pragma unroll
             for (int m = 0; m < NF; ++m) {
                 const double fi = f_inf(g + G * m);
-                val[m] = fi + (val[m] - fi) * rin / rgh;
+                val[m] = fi + quotient((val[m] - fi) * rin, rgh, inv);
             }
         }
     }
@@ -1113,7 +1130,7 @@ __device__ void fill_ghost_cell(const BlockDesc& b, gdouble* u, long t_, int mod
 }
 
 template <int G>
-__global__ void fill_ghosts_kernel(BlockDesc b, double* u, int mode, int faces) {
+__global__ __launch_bounds__(GHOST_WG) void fill_ghosts_kernel(BlockDesc b, double* u, int mode, int faces) {
     const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= ghost_count(b)) return;
     fill_ghost_cell<G>(b, (gdouble*)u, t, mode, faces, blockIdx.y);
@@ -1302,7 +1319,7 @@ __global__ void restrict_kernel(BlockDesc f, const double* __restrict__ fu, Bloc
 // every ghost cell of buffer `sel` of every block of a table; ofs[i] = first ghost cell of
 // block i (nblocks + 1 entries)
 template <int G>
-__global__ void fill_ghosts_batch_kernel(const BatchBlock* __restrict__ table, const int* __restrict__ wg_block,
+__global__ __launch_bounds__(GHOST_WG) void fill_ghosts_batch_kernel(const BatchBlock* __restrict__ table, const int* __restrict__ wg_block,
                                          int sel, int mode) {
     const BatchBlock& B = table[wg_block[blockIdx.x]]; // one block per workgroup
     const long t = (long)(blockIdx.x - B.ghost_wg0) * GHOST_WG + threadIdx.x;
