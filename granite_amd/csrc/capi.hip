@@ -10,7 +10,10 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
+#include <atomic>
 #include <cmath>
+#include <condition_variable>
 #include <cstdio>
 #include <fstream>
 #include <map>
@@ -24,6 +27,7 @@
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <utility>
 #include <vector>
 
@@ -58,6 +62,9 @@ struct gr_engine {
     size_t cap_src = 0;
     double* d_aux = nullptr;
     size_t cap_aux = 0;
+    double* h_stage = nullptr; // pinned host staging of the right-hand side call (doubles)
+    size_t cap_stage = 0;
+    std::vector<hipEvent_t> stage_events;
 };
 
 // Blocks of a level that share one grid spacing bit for bit: one stage launch (the stencil
@@ -246,6 +253,8 @@ int gr_engine_destroy(gr_engine* e) {
     if (e->d_r) (void)hipFree(e->d_r);
     if (e->d_src) (void)hipFree(e->d_src);
     if (e->d_aux) (void)hipFree(e->d_aux);
+    if (e->h_stage) (void)hipHostFree(e->h_stage);
+    for (hipEvent_t ev : e->stage_events) (void)hipEventDestroy(ev);
     if (e->aux.stream) (void)hipStreamSynchronize(e->aux.stream);
     if (e->aux.fork) (void)hipEventDestroy(e->aux.fork);
     if (e->aux.join) (void)hipEventDestroy(e->aux.join);
@@ -271,6 +280,151 @@ int gr_engine_sync(gr_engine* e) {
     return GR_OK;
 }
 
+} // extern "C"
+
+namespace {
+
+// The host call of the right-hand side moves the state in and the interior of the result out,
+// through pinned memory that several threads fill and empty beside the copies; the caller's
+// ghost cells of the result are not touched, so they are not sent either.
+// Three direct copies of pageable memory (state in, result in for its ghosts, result out) against
+// this, us: 12^3 223 -> 126, 24^3 697 -> 330, 48^3 3940 -> 1545, 80^3 15300 -> 5200. Pinned memory
+// is bounded; a block above the bound (90^3 and more) keeps the direct copies, as does memory
+// that the host cannot read by itself.
+constexpr size_t kStageMaxBytes = 128u << 20;     // larger blocks keep the direct copies
+constexpr size_t kStageBytesPerThread = 4u << 20; // a thread more per 4 MiB of state ..
+constexpr int kStageMaxThreads = 8;               // .. up to 8
+constexpr int kStageChunks = 11;                  // of two fields each with several threads, else one
+
+// whether p is memory the host can copy by itself (not device memory)
+bool host_readable(const void* p) {
+    hipPointerAttribute_t a;
+    if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+        (void)hipGetLastError(); // not known to the runtime: ordinary host memory
+        return true;
+    }
+    return a.type == hipMemoryTypeHost || a.type == hipMemoryTypeUnregistered;
+}
+
+// pinned staging for n doubles and the chunks' events; false: not to be had, use direct copies
+bool stage_ready(gr_engine* e, size_t n) {
+    if (n * sizeof(double) > kStageMaxBytes) return false;
+    while (e->stage_events.size() < (size_t)kStageChunks) {
+        hipEvent_t ev = nullptr;
+        if (hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess) {
+            (void)hipGetLastError();
+            return false;
+        }
+        e->stage_events.push_back(ev);
+    }
+    if (e->cap_stage >= n) return true;
+    if (e->h_stage) (void)hipHostFree(e->h_stage);
+    e->h_stage = nullptr;
+    e->cap_stage = 0;
+    if (hipHostMalloc((void**)&e->h_stage, n * sizeof(double), hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        e->h_stage = nullptr;
+        return false;
+    }
+    e->cap_stage = n;
+    return true;
+}
+
+struct StagedRhs {
+    gr_engine* e;
+    const gr::BlockDesc& b;
+    const double* u;
+    double* rhs;
+    std::atomic<int> in{0}, out{0};       // next field to send, next chunk to scatter
+    std::atomic<int> status{hipSuccess};  // first error of any thread
+    std::mutex m;
+    std::condition_variable cv;
+    int chunks = 1;  // of the result
+    int sent = 0;    // helpers done with the state
+    bool go = false; // the result's copies are enqueued (or failed: status)
+
+    void note(hipError_t st) {
+        int ok = hipSuccess;
+        if (st != hipSuccess) status.compare_exchange_strong(ok, (int)st);
+    }
+    void send() {
+        for (int v; (v = in.fetch_add(1)) < 22;) {
+            const size_t o = (size_t)v * b.stride;
+            std::memcpy(e->h_stage + o, u + o, b.stride * sizeof(double));
+            note(hipMemcpyAsync(e->d_u + o, e->h_stage + o, b.stride * sizeof(double), hipMemcpyHostToDevice, e->stream));
+        }
+    }
+    void scatter() {
+        const long ncell = (long)b.n[0] * b.n[1] * b.n[2];
+        for (int c; (c = out.fetch_add(1)) < chunks && status == hipSuccess;) {
+            const hipError_t st = hipEventSynchronize(e->stage_events[c]);
+            note(st);
+            if (st != hipSuccess) return;
+            for (int v = c * (22 / chunks); v < (c + 1) * (22 / chunks); ++v) {
+                const double* p = e->h_stage + v * ncell;
+                for (int k = 0; k < b.n[2]; ++k)
+                    for (int j = 0; j < b.n[1]; ++j, p += b.n[0])
+                        std::memcpy(rhs + (size_t)v * b.stride + b.ng +
+                                        (size_t)b.nt[0] * ((b.ng + j) + (size_t)b.nt[1] * (b.ng + k)),
+                                    p, b.n[0] * sizeof(double));
+            }
+        }
+    }
+    void help() {
+        note(hipSetDevice(e->device));
+        send();
+        {
+            std::unique_lock<std::mutex> l(m);
+            ++sent;
+            cv.notify_all();
+            cv.wait(l, [&] { return go; });
+        }
+        scatter();
+    }
+    // launch(): the kernel from d_u into d_r, on the engine's stream
+    template <class F>
+    hipError_t run(F&& launch) {
+        const size_t bytes = 22 * (size_t)b.stride * sizeof(double), ncell = (size_t)b.n[0] * b.n[1] * b.n[2];
+        const int want = (int)std::min<size_t>(kStageMaxThreads, bytes / kStageBytesPerThread);
+        std::array<std::thread, kStageMaxThreads> t;
+        int helpers = 0;
+        try {
+            for (; helpers + 1 < want; ++helpers) t[helpers] = std::thread([this] { help(); });
+        } catch (...) { // no thread to be had: the calling one does the rest
+        }
+        if (helpers)
+            send();
+        else
+            note(hipMemcpyAsync(e->d_u, u, bytes, hipMemcpyHostToDevice, e->stream));
+        {
+            std::unique_lock<std::mutex> l(m);
+            cv.wait(l, [&] { return sent == helpers; });
+        }
+        if (status == hipSuccess) note(launch());
+        if (status == hipSuccess) note(gr::launch_pack_interior(b, e->d_r, e->d_u, e->stream));
+        chunks = helpers ? kStageChunks : 1;
+        const size_t len = 22 / chunks * ncell;
+        for (int c = 0; c < chunks && status == hipSuccess; ++c) {
+            const size_t o = c * len;
+            note(hipMemcpyAsync(e->h_stage + o, e->d_u + o, len * sizeof(double), hipMemcpyDeviceToHost, e->stream));
+            note(hipEventRecord(e->stage_events[c], e->stream));
+        }
+        {
+            std::lock_guard<std::mutex> l(m);
+            go = true;
+            cv.notify_all();
+        }
+        scatter();
+        for (int h = 0; h < helpers; ++h) t[h].join();
+        note(hipStreamSynchronize(e->stream));
+        return (hipError_t)status.load();
+    }
+};
+
+} // namespace
+
+extern "C" {
+
 int gr_ccz4_rhs(gr_engine* e, const gr_geom* geom, const gr_ccz4_params* prm, int nvars, const double* u,
                 double* rhs, const double* rho, const double* Si, const double* Sij, const double* S) {
     int rc = use_device(e);
@@ -295,12 +449,20 @@ int gr_ccz4_rhs(gr_engine* e, const gr_geom* geom, const gr_ccz4_params* prm, in
         GR_HIP(e, hipMemcpyAsync(d + 10 * b.stride, S, b.stride * sizeof(double), hipMemcpyHostToDevice, e->stream));
         src = gr::Sources{d, d + b.stride, d + 4 * b.stride, d + 10 * b.stride};
     }
+    static const int sel[3] = {0, 1, 2};
+    auto launch = [&] {
+        return gr::launch_stage_fp64(gr::single_batch(b, e->d_u, e->d_u, e->d_r, src), sel, src.rho != nullptr,
+                                     cell_params(prm), prm->ko_sigma, gr::MODE_RHS, gr::StageCoef{0.0, 0.0, 0.0},
+                                     e->stream);
+    };
+    if (host_readable(u) && host_readable(rhs) && stage_ready(e, n)) {
+        StagedRhs call{e, b, u, rhs};
+        GR_HIP(e, call.run(launch));
+        return GR_OK;
+    }
     GR_HIP(e, hipMemcpyAsync(e->d_u, u, n * sizeof(double), hipMemcpyHostToDevice, e->stream));
     GR_HIP(e, hipMemcpyAsync(e->d_r, rhs, n * sizeof(double), hipMemcpyHostToDevice, e->stream));
-    static const int sel[3] = {0, 1, 2};
-    GR_HIP(e, gr::launch_stage_fp64(gr::single_batch(b, e->d_u, e->d_u, e->d_r, src), sel, src.rho != nullptr,
-                                    cell_params(prm), prm->ko_sigma, gr::MODE_RHS, gr::StageCoef{0.0, 0.0, 0.0},
-                                    e->stream));
+    GR_HIP(e, launch());
     GR_HIP(e, hipMemcpyAsync(rhs, e->d_r, n * sizeof(double), hipMemcpyDeviceToHost, e->stream));
     GR_HIP(e, hipStreamSynchronize(e->stream));
     return GR_OK;

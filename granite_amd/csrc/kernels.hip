@@ -1039,8 +1039,8 @@ __device__ __forceinline__ long ghost_count(const BlockDesc& b) {
 // (src/amr/amr.cpp:412-480).
 // Fields g, g + G, ... of the cell: the G field groups run as separate workgroups (second
 // grid dimension), so a small ghost region still fills the machine.
-// Bound by memory: at 192^3 91 us for 145 MB read and 159 MB written, 56 us of them (6 of these the
-// launch's) the x columns, which read two 64-byte lines and write one per row end and field. With
+// Bound by memory: at 192^3 91 us for 290 MB read and 159 MB written, 4.9 TB/s, 56 us of them (6 of
+// these the launch's) the x columns, whose anchors cost a 128-byte line per row end and field. With
 // the division by a shared reciprocal and each such line written by neighbouring lanes at once:
 // 192^3 95 -> 91 us, 128^3 42.4 -> 40.7, the 64 uneven blocks (four launches) 206 -> 199.
 template <int G>
@@ -1314,6 +1314,17 @@ __global__ void restrict_kernel(BlockDesc f, const double* __restrict__ fu, Bloc
                 for (int ri = 0; ri < 2; ++ri) s += F[(b[0] + ri) + (long)f.nt[0] * ((b[1] + rj) + (long)f.nt[1] * (b[2] + rk))];
         cu[v * c.stride + dst] = s / 8;
     }
+}
+
+// interior cells of `r`, field by field, without the ghosts between them
+__global__ void pack_interior_kernel(BlockDesc b, const double* __restrict__ r, double* __restrict__ out) {
+    const int t = (int)(blockIdx.x * blockDim.x + threadIdx.x); // interior cells < 2^29
+    const int ncell = b.n[0] * b.n[1] * b.n[2];
+    if (t >= ncell) return;
+    const int i = t % b.n[0], q = t / b.n[0], j = q % b.n[1], k = q / b.n[1];
+    const long src = (b.ng + i) + (long)b.nt[0] * ((b.ng + j) + (long)b.nt[1] * (b.ng + k));
+    const int v = blockIdx.y;
+    out[(long)v * ncell + t] = r[v * b.stride + src];
 }
 
 // every ghost cell of buffer `sel` of every block of a table; ofs[i] = first ghost cell of
@@ -2067,6 +2078,12 @@ hipError_t launch_restrict(const BlockDesc& f, const double* fu, const BlockDesc
     const long n = (long)c.n[0] * c.n[1] * c.n[2];
     const int g = groups > 0 && groups <= NV ? groups : GR_TRANSFER_GROUPS;
     restrict_kernel<<<dim3(grid_for(n, 256), g), 256, 0, s>>>(f, fu, c, cu);
+    return hipGetLastError();
+}
+
+hipError_t launch_pack_interior(const BlockDesc& b, const double* r, double* out, hipStream_t s) {
+    const long n = (long)b.n[0] * b.n[1] * b.n[2];
+    pack_interior_kernel<<<dim3(grid_for(n, 256), NV), 256, 0, s>>>(b, r, out);
     return hipGetLastError();
 }
 

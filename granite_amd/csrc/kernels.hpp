@@ -139,6 +139,9 @@ hipError_t launch_prolongate(const BlockDesc& c, const double* cu, const BlockDe
 hipError_t launch_restrict(const BlockDesc& f, const double* fu, const BlockDesc& c, double* cu, hipStream_t s,
                            int groups = 0);
 
+// out = the interior cells of all 22 fields of r, field by field (k, j, i)
+hipError_t launch_pack_interior(const BlockDesc& b, const double* r, double* out, hipStream_t s);
+
 // rhs += Kreiss-Oliger(u) on the interior (reference accumulation order)
 hipError_t launch_dissipation(const BlockDesc& b, const double* u, double* rhs, double ko_sigma, hipStream_t s);
 
