@@ -11,8 +11,8 @@
 #include <cstdint>
 
 // tile shape (overridable at build time): a tile of GR_TILE_X x Y x Z cells is the unit of
-// the launch bookkeeping and of the mixed-precision classification and kernel (one thread
-// per cell); the FP64 kernel runs each tile as parts (FP64_PARTS below)
+// the launch bookkeeping and of the mixed form's choice of precision; the kernels run each tile as
+// parts (FP64_PARTS below), one thread per cell
 #ifndef GR_TILE_X
 #define GR_TILE_X 16
 #endif
@@ -24,19 +24,6 @@
 #endif
 #ifndef GR_FP64_KO_EXACT
 #define GR_FP64_KO_EXACT 1
-#endif
-// parts of a tile along x the mixed kernel runs as separate workgroups (1 or 2)
-#ifndef GR_MIXED_SPLIT
-#define GR_MIXED_SPLIT 1
-#endif
-#ifndef GR_MIXED_MIN_WAVES
-#define GR_MIXED_MIN_WAVES 1
-#endif
-#ifndef GR_MIXED_PREFETCH
-#define GR_MIXED_PREFETCH 1
-#endif
-#ifndef GR_LDS_PAD32
-#define GR_LDS_PAD32 1
 #endif
 // default field groups (second grid dimension) of the ghost fill (1, 2, 4 or 11)
 #ifndef GR_GHOST_GROUPS
@@ -114,37 +101,9 @@ __device__ __forceinline__ void algebraic_exact(double g[6], double A[6]) {
 }
 
 // ------------------------------------------------------------------------------------
-// FP32 LDS staging of one field of a tile (the mixed form)
+// parts of a tile and their LDS boxes
 // ------------------------------------------------------------------------------------
-// Smallest LDS row pitch >= bx0 (elements of esize bytes, rows of a box by rows high) at
-// which the 64 lanes of a wave, laid over the tile x fastest, then y, then z, read their
-// cells without bank conflicts. The LDS serves 64 four-byte banks per pass, so a wave's
-// read of esize-byte elements takes esize / 4 passes of 256 / esize consecutive lanes, each
-// conflict-free when its words fall on distinct banks. The stencil taps shift all lanes
-// alike, so they inherit the pattern of the centre read.
-template <int TX, int TY>
-constexpr int conflict_free_pitch(int bx0, int by, int esize) {
-    const int words = esize / 4, lanes = 64 / words;
-    for (int p = bx0; p < bx0 + 64; ++p) {
-        bool clean = true;
-        for (int pass = 0; pass < words && clean; ++pass) {
-            bool used[64] = {};
-            for (int t = pass * lanes; t < (pass + 1) * lanes && clean; ++t) {
-                const int lx = t % TX, ly = (t / TX) % TY, lz = t / (TX * TY);
-                const int a = (lz * by + ly) * p + lx;
-                for (int w = 0; w < words; ++w) {
-                    const int bank = (a * words + w) % 64;
-                    clean = clean && !used[bank];
-                    used[bank] = true;
-                }
-            }
-        }
-        if (clean) return p;
-    }
-    return bx0;
-}
-
-// Lane -> cell map of the FP64 parts (16 x 4 x TZ): lane bits 0-3 are x, bit 4 the low bit of z, bit
+// Lane -> cell map of the parts (16 x 4 x TZ): lane bits 0-3 are x, bit 4 the low bit of z, bit
 // 5 the low bit of y, and the wave index supplies the rest of y, then of z. A 64-bit read then
 // takes each 16-lane group from one row and the 32 lanes of two groups from two planes, which
 // are conflict-free where a plane spans 16 doubles modulo 32.
@@ -175,51 +134,6 @@ constexpr bool lds_conflict_free(int P, int Q) {
         }
     return true;
 }
-
-template <int TX, int TY, int TZ, bool PAD = true>
-struct TileGeom {
-    static constexpr int NT = TX * TY * TZ;
-    static constexpr int BX0 = TX + 2 * HALO, BY = TY + 2 * HALO, BZ = TZ + 2 * HALO;
-    // LDS row pitch and plane stride (floats): conflict-free centre reads
-    static constexpr int BX = PAD ? conflict_free_pitch<TX, TY>(BX0, BY, 4) : BX0;
-    static constexpr int PLANE = BX * BY;
-    static constexpr int NLDS = PLANE * BZ;
-    // sub-boxes of the halo region that some stencil reads (x0,x1,y0,y1,z0,z1)
-    static constexpr int NBOX = 7;
-    static constexpr int box[NBOX][6] = {
-        {-HALO, TX + HALO, 0, TY, 0, TZ},          // tile + x halo
-        {-1, TX + 1, -HALO, 0, 0, TZ},             // y halo (low) with the xy edge column
-        {-1, TX + 1, TY, TY + HALO, 0, TZ},        // y halo (high)
-        {-1, TX + 1, -1, TY + 1, -1, 0},           // z = -1 layer with xz / yz edges
-        {-1, TX + 1, -1, TY + 1, TZ, TZ + 1},      // z = TZ layer
-        {0, TX, 0, TY, -HALO, -1},                 // z halo (low), axis taps only
-        {0, TX, 0, TY, TZ + 1, TZ + HALO},         // z halo (high)
-    };
-    static constexpr int count(int b) {
-        return (box[b][1] - box[b][0]) * (box[b][3] - box[b][2]) * (box[b][5] - box[b][4]);
-    }
-    static constexpr int start(int b) { return b == 0 ? 0 : start(b - 1) + count(b - 1); }
-    static constexpr int TOTAL = start(NBOX - 1) + count(NBOX - 1);
-    __host__ __device__ static constexpr int lds(int x, int y, int z) {
-        return (z + HALO) * PLANE + (y + HALO) * BX + (x + HALO);
-    }
-    // tile-relative coordinates of halo entry p (boxes in order, x fastest inside a box);
-    // unchanged for p >= TOTAL. The boxes are visited at compile time, so their extents
-    // are immediates and the divisions constant.
-    template <int K = 0>
-    __device__ static void entry(int p, int& x, int& y, int& z) {
-        if constexpr (K < NBOX) {
-            constexpr int nx = box[K][1] - box[K][0], ny = box[K][3] - box[K][2];
-            const int q = p - start(K);
-            if (q >= 0 && q < count(K)) {
-                x = box[K][0] + q % nx;
-                y = box[K][2] + (q / nx) % ny;
-                z = box[K][4] + q / (nx * ny);
-            }
-            entry<K + 1>(p, x, y, z);
-        }
-    }
-};
 
 // LDS layout of one field's halo box of a 16 x 4 x TZ part: little more than what some stencil
 // reads. Planes z = -1 .. TZ lie one after the other in 12 rows of 24 doubles (x = -4 .. 19) and 16
@@ -309,9 +223,9 @@ struct PackedBox {
 // the planes next to it, each near enough for the paired LDS reads' 8-bit offsets: from the cell
 // itself the compiler adds an address for nearly every pair, 228 instructions a part (128^3,
 // stages 1-2: 504 -> 497 us; the uneven 64 blocks 772 -> 762).
-template <class Box>
+template <class Box, typename R>
 struct PackedTaps {
-    typedef const __attribute__((address_space(3))) double* LdsPtr;
+    typedef const __attribute__((address_space(3))) R* LdsPtr;
     static constexpr int NB = 4; // buffers, at most
     LdsPtr z[6];        // z - 4, - 3, - 2, + 2, + 3, + 4 in buffer 0
     LdsPtr base[NB][3]; // per buffer: planes z - 1, z, z + 1
@@ -335,14 +249,14 @@ struct PackedTaps {
 #endif
             }
     }
-    __device__ __forceinline__ double near(int dz, int q) const { return base[buf][dz + 1][q - low(dz + 1) + dz * Box::PL]; }
-    __device__ __forceinline__ double at(const double*, int d, int k) const {
+    __device__ __forceinline__ R near(int dz, int q) const { return base[buf][dz + 1][q - low(dz + 1) + dz * Box::PL]; }
+    __device__ __forceinline__ R at(const R*, int d, int k) const {
         if (d == 2 && (k >= 2 || k <= -2)) return z[k < 0 ? k + 4 : k + 1][ofs];
         return d == 2 ? near(k, 0) : near(0, d == 1 ? k * Box::ROW : k);
     }
-    __device__ __forceinline__ double centre(const double*) const { return near(0, 0); }
+    __device__ __forceinline__ R centre(const R*) const { return near(0, 0); }
     // i cells along axis a and j along axis b > a (i, j = -1 or 1)
-    __device__ __forceinline__ double edge(const double*, int a, int b, int i, int j) const {
+    __device__ __forceinline__ R edge(const R*, int a, int b, int i, int j) const {
         const int q = a == 0 ? i : i * Box::ROW;
         return b == 2 ? near(j, q) : near(0, q + j * Box::ROW);
     }
@@ -367,6 +281,15 @@ struct MonitorOrder {
         return p;
     }
 };
+
+// byte offset of the pair at (x, y, z) of the part, or of the part's first pair where it lies
+// beyond the block (a pair at the end of an odd row takes the next row's first cell along)
+__device__ __forceinline__ unsigned pair_offset(int x, int y, int z, int ox, int oy, int oz, const BlockDesc& b) {
+    const int gx = ox + x, gy = oy + y, gz = oz + z;
+    const int i = gx + b.nt[0] * (gy + b.nt[1] * gz);
+    const bool ok = gx < b.nt[0] && gy < b.nt[1] && gz < b.nt[2] && i + 1 < b.nt[0] * b.nt[1] * b.nt[2];
+    return 8u * (unsigned)(ok ? i : ox + b.nt[0] * (oy + b.nt[1] * oz));
+}
 
 // Per-thread input/output of one cell of an FP64 part: stages the fields into LDS for the
 // stencils (Stager interface of ccz4_cell) and combines/stores the results (Sink interface).
@@ -434,21 +357,12 @@ struct TileIODma {
     unsigned doff[KW]; // byte offset of this lane's pair in each of its wave's chunks
     unsigned uoff; // byte offset of the u^n pair this lane stages (lanes 0-31: the wave's 64 cells)
     int tid;
-    PackedTaps<Box> taps;
+    PackedTaps<Box, double> taps;
     double unA[6]; // u^n of A~, whose results come after the last field
     double hA[6];
 
     __device__ __forceinline__ void place(int lx, int ly, int lz) {
         taps.place((LdsPtr)lds + BUF0, lx, ly, lz, NBUF, LBUF);
-    }
-
-    // byte offset of the pair at (x, y, z) of the part, or of the part's first pair where it lies
-    // beyond the block (a pair at the end of an odd row takes the next row's first cell along)
-    __device__ __forceinline__ unsigned pair_offset(int x, int y, int z, int ox, int oy, int oz, const BlockDesc& b) const {
-        const int gx = ox + x, gy = oy + y, gz = oz + z;
-        const int i = gx + b.nt[0] * (gy + b.nt[1] * gz);
-        const bool ok = gx < b.nt[0] && gy < b.nt[1] && gz < b.nt[2] && i + 1 < b.nt[0] * b.nt[1] * b.nt[2];
-        return 8u * (unsigned)(ok ? i : ox + b.nt[0] * (oy + b.nt[1] * oz));
     }
 
     __device__ void init(int tid_, int ox, int oy, int oz, const BlockDesc& b) {
@@ -518,7 +432,7 @@ struct TileIODma {
 #pragma unroll
         for (int a = 0; a < 6; ++a) g[a] = gload(in + (GXX + a) * stride, cb);
     }
-    __device__ const PackedTaps<Box>& strides() const { return taps; }
+    __device__ const PackedTaps<Box, double>& strides() const { return taps; }
     __device__ const double* field(int v) {
         const int pos = Order::pos(v);
         // this wave's loads of field pos have landed and its LDS accesses are done; then the
@@ -583,72 +497,80 @@ struct TileIODma {
 // tile (the field at the tile's first cell): every stencil's weights sum to zero, so
 // derivatives of the deltas are derivatives of the field, while small structure on top of
 // an O(1) field (1e-8 noise on the metric) keeps FP32 relative precision of the delta.
+// The box is the packed one of the FP64 parts in floats, filled through registers one field ahead (the
+// deltas are formed on the way), by the pairs each lane would load directly: four 16-byte loads
+// and four 8-byte LDS writes a thread and field. 16x4x4 parts of 256 threads against whole 16x4x8
+// tiles of 512 with a box of single values and its corners (one workgroup per CU): two independent
+// workgroups per CU or, with the FP64 tiles beside them, one (128^3: stages 1-2 516 -> 485 us,
+// stage 3 557 -> 521; 192^3 1665 -> 1551, 1800 -> 1673). At three waves per SIMD (168 registers) stage
+// 3 gains 2% at 128^3 and loses 7% at 101x77x59, where FP64 tiles are a larger share.
 // UN_IN: u^n is the stage input itself (the first stage, chosen at launch): its value at the
 // cell is the stage input's centre value, so it is not loaded separately
-template <int TX, int TY, int TZ, int MODE, int PF, bool UN_IN = false>
+template <int TZ, int MODE, bool UN_IN = false>
 struct TileIO32 {
-    using T = TileGeom<TX, TY, TZ, GR_LDS_PAD32 != 0>;
-    static constexpr int NL = (T::TOTAL + T::NT - 1) / T::NT;
-    static constexpr int LBUF = T::NLDS + 1;
+    using Box = PackedBox<TZ>;
+    typedef __attribute__((address_space(3))) float* LdsPtr;
+    typedef double pair __attribute__((ext_vector_type(2), aligned(8)));
+    typedef float pair32 __attribute__((ext_vector_type(2)));
+    static constexpr int NT = Box::TX * Box::TY * TZ, CH = 128, NCH = (Box::SIZE + CH - 1) / CH;
+    static constexpr int LBUF = NCH * CH, KW = NCH / (NT / 64);
+    static_assert(Box::consistent() && NCH % (NT / 64) == 0, "packed box, the same number of chunks for each wave");
 
     float* lds; // 2 * LBUF floats
     const gdouble* in; // global address space: loads/stores wait on vmcnt only, never on LDS waits
     const gdouble* un;
     gdouble* out;
     long stride;
-    long cidx;
     unsigned cb; // byte offset of the thread's cell inside one field
     long ridx; // the tile's reference cell
-    int cl;
     bool active;
     bool ko_on;
     StageCoef cf;
-    int loff[NL];
-    unsigned goff[NL];
-    double buf[PF][NL];
-    double refb[PF], unb[PF], inb[PF];
+    int tid;
+    unsigned doff[KW]; // byte offset of the thread's pairs of the halo box
+    PackedTaps<Box, float> taps;
+    pair buf[KW];
+    double refb, unb, inb;
     double unv[NV], inv[NV];
-    double hg[6], hA[6];
+    double* metric; // last stage: the new metric waits in LDS (6 * NT doubles) for the algebraic constraints
+    double hA[6];
 
-    __device__ void init(int tid, int ox, int oy, int oz, int nt0, int nt1, int nt2) {
+    __device__ void init(int tid_, int lx, int ly, int lz, int ox, int oy, int oz, const BlockDesc& b) {
+        tid = tid_;
+        taps.place((LdsPtr)lds, lx, ly, lz, 2, LBUF);
 #pragma unroll
-        for (int i = 0; i < NL; ++i) {
-            const int p = tid + i * T::NT;
+        for (int k = 0; k < KW; ++k) {
             int x = 0, y = 0, z = 0;
-            T::entry(p, x, y, z);
-            const int gx = ox + x, gy = oy + y, gz = oz + z;
-            const bool ok = p < T::TOTAL && gx < nt0 && gy < nt1 && gz < nt2;
-            loff[i] = ok ? T::lds(x, y, z) : T::NLDS;
-            goff[i] = ok ? 8u * (unsigned)(gx + nt0 * (gy + nt1 * gz)) : 0u;
+            Box::point(2 * (tid + k * NT), x, y, z);
+            doff[k] = pair_offset(x, y, z, ox, oy, oz, b);
         }
-#pragma unroll
-        for (int k = 0; k < PF; ++k) prefetch(k);
+        prefetch(0);
         stage_to_lds(0);
-        prefetch(PF);
+        prefetch(1);
     }
 
     __device__ __forceinline__ void prefetch(int pos) {
         if (pos >= NV) return;
         const int v = FIELD_ORDER[pos];
-        const int slot = pos % PF;
         const gdouble* f = in + v * stride;
 #pragma unroll
-        for (int i = 0; i < NL; ++i) buf[slot][i] = gload(f, goff[i]);
-        refb[slot] = f[ridx];
-        inb[slot] = gload(f, cb);
-        if (MODE != MODE_RHS && !UN_IN) unb[slot] = gload(un + v * stride, cb);
+        for (int k = 0; k < KW; ++k)
+            buf[k] = *(const __attribute__((address_space(1))) pair*)((const gchar*)f + doff[k]);
+        refb = f[ridx];
+        inb = gload(f, cb);
+        if (MODE != MODE_RHS && !UN_IN) unb = gload(un + v * stride, cb);
     }
 
     __device__ __forceinline__ void stage_to_lds(int pos) {
         if (pos >= NV) return;
-        const int slot = pos % PF;
         float* L = lds + (pos & 1) * LBUF;
-        const double r = refb[slot];
+        const double r = refb;
 #pragma unroll
-        for (int i = 0; i < NL; ++i) L[loff[i]] = (float)(buf[slot][i] - r);
+        for (int k = 0; k < KW; ++k)
+            *(pair32*)(L + 2 * (tid + k * NT)) = pair32{(float)(buf[k].x - r), (float)(buf[k].y - r)};
         const int v = FIELD_ORDER[pos];
-        inv[v] = inb[slot];
-        if (MODE != MODE_RHS) unv[v] = UN_IN ? inb[slot] : unb[slot];
+        inv[v] = inb;
+        if (MODE != MODE_RHS) unv[v] = UN_IN ? inb : unb;
     }
 
     // ---- Stager
@@ -657,13 +579,15 @@ struct TileIO32 {
 #pragma unroll
         for (int a = 0; a < 6; ++a) g[a] = gload(in + (GXX + a) * stride, cb);
     }
-    __device__ FixedStrides<1, T::BX, T::PLANE> strides() const { return {}; }
+    __device__ const PackedTaps<Box, float>& strides() const { return taps; }
     __device__ const float* field(int v) {
         const int pos = field_pos(v);
         __syncthreads();
         stage_to_lds(pos + 1);
-        prefetch(pos + 1 + PF);
-        return lds + (pos & 1) * LBUF + cl;
+        prefetch(pos + 2);
+        taps.buf = pos & 1;
+        taps.ofs = (pos & 1) * LBUF;
+        return lds; // the taps know the cell
     }
 
     // ---- Sink (FP64 combine on the FP64 stage input and u^n)
@@ -677,7 +601,7 @@ struct TileIO32 {
         if (v == CHI) val = floor_chi(val);
         if (v == ALPHA) val = floor_alpha(val);
         if (MODE == MODE_FINAL && v >= GXX && v < GXX + 6) {
-            hg[v - GXX] = val;
+            metric[(v - GXX) * NT + tid] = val;
             return;
         }
         if (MODE == MODE_FINAL && v >= AXX && v < AXX + 6) {
@@ -689,6 +613,9 @@ struct TileIO32 {
 
     __device__ __forceinline__ void finish() {
         if (MODE != MODE_FINAL) return;
+        double hg[6];
+#pragma unroll
+        for (int a = 0; a < 6; ++a) hg[a] = metric[a * NT + tid];
         algebraic_exact(hg, hA);
         if (!active) return;
 #pragma unroll
@@ -872,8 +799,11 @@ __global__ __launch_bounds__(64 * TZ, TZ / 2) void stage_kernel(StageArgs A) {
     stage_tile<TZ, MODE, HAS_SRC, KO_EXACT, UN_IN>(A, R, part, lds);
 }
 
-// the flagged tiles only, from a small grid: each workgroup gathers the tiles with
-// flags == want among tiles blockIdx.x + k * gridDim.x and runs them one after the other
+// the parts of the flagged tiles only, from a small grid: each workgroup gathers those with
+// flags == want among parts blockIdx.x + k * gridDim.x and runs them one after the other. By part
+// and not by tile, so that the parts of a tile run beside each other: small blocks, whose few FP64
+// tiles take longer than all others, wait for one part instead of two (with the FP32 parts, mixed
+// 32^3 step 244 -> 196 us, 64^3 332 -> 292, 101x77x59 711 -> 620).
 // (every thread takes the same trip counts, so the barriers are uniform)
 template <int TZ, int MODE, bool HAS_SRC, bool KO_EXACT, bool UN_IN>
 __global__ __launch_bounds__(64 * TZ) void stage_kernel_scan(StageArgs A) {
@@ -881,22 +811,22 @@ __global__ __launch_bounds__(64 * TZ) void stage_kernel_scan(StageArgs A) {
     __shared__ __align__(16) double lds[TileIODma<TZ, MODE, UN_IN>::LDS_DOUBLES];
     __shared__ int list[NT];
     __shared__ int nlist;
-    const int per = (int)gridDim.x * NT;
-    for (int base = 0; base < A.ntiles; base += per) {
+    constexpr int NP = FP64_PARTS<TZ>;
+    const int per = (int)gridDim.x * NT, nparts = A.ntiles * NP;
+    for (int base = 0; base < nparts; base += per) {
         if (threadIdx.x == 0) nlist = 0;
         __syncthreads();
         const int t = base + (int)blockIdx.x + (int)threadIdx.x * (int)gridDim.x;
-        if (t < A.ntiles && A.flags[t] == A.want) list[atomicAdd(&nlist, 1)] = t;
+        if (t < nparts && A.flags[t / NP] == A.want) list[atomicAdd(&nlist, 1)] = t;
         __syncthreads();
         const int n = nlist;
         __syncthreads();
         for (int item = 0; item < n; ++item) {
-            const TileRef R = resolve_tile(A, list[item]);
-            for (int part = 0; part < FP64_PARTS<TZ>; ++part) {
-                if (part_outside<TZ>(R, part)) continue; // uniform over the workgroup
-                stage_tile<TZ, MODE, HAS_SRC, KO_EXACT, UN_IN>(A, R, part, lds);
-                __syncthreads(); // the next part reuses the LDS buffers
-            }
+            const int unit = list[item], part = unit % NP;
+            const TileRef R = resolve_tile(A, unit / NP);
+            if (part_outside<TZ>(R, part)) continue; // uniform over the workgroup
+            stage_tile<TZ, MODE, HAS_SRC, KO_EXACT, UN_IN>(A, R, part, lds);
+            __syncthreads(); // the next part reuses the LDS buffers
         }
     }
 }
@@ -911,43 +841,43 @@ constexpr int LARGE_TILES = 256 / FP64_PARTS<TZ_SMALL> + 1; // small parts outnu
 // workgroups of the FP64 pass of the mixed form: one per CU
 constexpr int FP64_SCAN_GRID = 256;
 
-// one part of TX x TY x TZ cells (TILE_X / TX parts along x) of a launch tile per workgroup;
-// the tile is the unit of the FP32 / FP64 choice
-template <int TX, int TY, int TZ, int MODE, bool HAS_SRC, bool UN_IN = false>
-__global__ __launch_bounds__(TX* TY* TZ, GR_MIXED_MIN_WAVES) void stage_kernel_mixed(StageArgs A) {
-    using T = TileGeom<TX, TY, TZ, GR_LDS_PAD32 != 0>;
-    constexpr int NP = GR_TILE_X / TX;
-    static_assert(GR_TILE_X % TX == 0 && TY == GR_TILE_Y && TZ == GR_TILE_Z, "parts split the tile along x");
-    __shared__ float lds[2 * (T::NLDS + 1)];
+// one part of TZ layers of a launch tile per workgroup; the tile is the unit of the FP32 / FP64
+// choice and of the reference value of the deltas
+template <int TZ, int MODE, bool HAS_SRC, bool UN_IN = false>
+__global__ __launch_bounds__(64 * TZ, 2) void stage_kernel_mixed(StageArgs A) {
+    using IO = TileIO32<TZ, MODE, UN_IN>;
+    constexpr int NP = FP64_PARTS<TZ>;
+    __shared__ __align__(16) float lds[2 * IO::LBUF];
+    __shared__ double metric[MODE == MODE_FINAL ? 6 * IO::NT : 1];
 
     const int slot = tile_of_block(blockIdx.x, A.ntiles * NP, A.xcd_remap);
     const int tile = slot / NP, part = slot % NP;
     if (A.flags && A.flags[tile] != A.want) return;
     const TileRef R = resolve_tile(A, tile);
+    if (part_outside<TZ>(R, part)) return; // whole workgroup, before any barrier
     const BlockDesc& b = R.b;
-    const int x0 = R.tix * GR_TILE_X + part * TX;
-    if (x0 >= b.n[0]) return; // whole workgroup, before any barrier
+    const int x0 = R.tix * TILE_X, y0 = R.tiy * TILE_Y, z0 = R.tiz * TILE_Z + part * TZ;
     const int tid = threadIdx.x;
-    const int lx = tid % TX, ly = (tid / TX) % TY, lz = tid / (TX * TY);
-    const int ix = x0 + lx, iy = R.tiy * TY + ly, iz = R.tiz * TZ + lz;
+    int lx = 0, ly = 0, lz = 0;
+    LaneMap<TZ>::cell(tid, lx, ly, lz);
+    const int ix = x0 + lx, iy = y0 + ly, iz = z0 + lz;
     const bool active = ix < b.n[0] && iy < b.n[1] && iz < b.n[2];
     const int gi = b.ng + (active ? ix : 0), gj = b.ng + (active ? iy : 0), gk = b.ng + (active ? iz : 0);
     const long cidx = gi + (long)b.nt[0] * (gj + (long)b.nt[1] * gk);
 
-    TileIO32<TX, TY, TZ, MODE, GR_MIXED_PREFETCH, UN_IN> io;
+    IO io;
     io.lds = lds;
+    io.metric = metric;
     io.in = R.in;
     io.un = R.un;
     io.out = R.out;
     io.stride = b.stride;
-    io.cidx = cidx;
     io.cb = 8u * (unsigned)cidx;
-    io.ridx = (b.ng + x0) + (long)b.nt[0] * ((b.ng + R.tiy * TY) + (long)b.nt[1] * (b.ng + R.tiz * TZ));
-    io.cl = T::lds(lx, ly, lz);
+    io.ridx = (b.ng + x0) + (long)b.nt[0] * ((b.ng + y0) + (long)b.nt[1] * (b.ng + R.tiz * TILE_Z));
     io.active = active;
     io.ko_on = A.ko_on != 0;
     io.cf = A.cf;
-    io.init(tid, b.ng + x0, b.ng + R.tiy * TY, b.ng + R.tiz * TZ, b.nt[0], b.nt[1], b.nt[2]);
+    io.init(tid, lx, ly, lz, b.ng + x0, b.ng + y0, b.ng + z0, b);
 
     CellSources src{};
     if (HAS_SRC) load_sources(R.src, cidx, src);
@@ -1964,7 +1894,8 @@ hipError_t launch_stage_fp64(const Batch& B, const int sel[3], bool has_src, con
     int nblk = 0;
     if (flags) {
         A.scan = 1;
-        nblk = A.ntiles < FP64_SCAN_GRID ? A.ntiles : FP64_SCAN_GRID;
+        nblk = A.ntiles * FP64_PARTS<TZ_LARGE>;
+        if (nblk > FP64_SCAN_GRID) nblk = FP64_SCAN_GRID;
     }
     if (has_src) {
         if (mode == MODE_RHS) return launch_stage_t<MODE_RHS, true>(A, nblk, large, s);
@@ -1978,15 +1909,13 @@ hipError_t launch_stage_fp64(const Batch& B, const int sel[3], bool has_src, con
 
 template <int MODE, bool HAS_SRC>
 static hipError_t launch_mixed_t(const StageArgs& A, hipStream_t s) {
-    constexpr int PX = TILE_X / GR_MIXED_SPLIT;
+    const dim3 grid(A.ntiles * FP64_PARTS<TZ_LARGE>), wg(64 * TZ_LARGE);
     // the first stage (u^n is the stage input) has an instance of its own, so that no load
     // of the kernel's register prefetch is conditional
     if (MODE == MODE_STAGE && A.sel_un == A.sel_in)
-        stage_kernel_mixed<PX, TILE_Y, TILE_Z, MODE, HAS_SRC, MODE == MODE_STAGE>
-            <<<dim3(A.ntiles * GR_MIXED_SPLIT), dim3(PX * TILE_Y * TILE_Z), 0, s>>>(A);
+        stage_kernel_mixed<TZ_LARGE, MODE, HAS_SRC, MODE == MODE_STAGE><<<grid, wg, 0, s>>>(A);
     else
-        stage_kernel_mixed<PX, TILE_Y, TILE_Z, MODE, HAS_SRC>
-            <<<dim3(A.ntiles * GR_MIXED_SPLIT), dim3(PX * TILE_Y * TILE_Z), 0, s>>>(A);
+        stage_kernel_mixed<TZ_LARGE, MODE, HAS_SRC><<<grid, wg, 0, s>>>(A);
     return hipGetLastError();
 }
 

@@ -182,7 +182,7 @@ hipError_t launch_init_gauge_wave(const BlockDesc& b, double* u, double A, doubl
 
 // tile shape of the FP64 stage kernel
 void stage_tile_fp64(int* t3);
-// tile of the launch bookkeeping and of the mixed-precision kernel (cells x, y, z)
+// tile of the launch bookkeeping and of the mixed form's choice of precision (cells x, y, z)
 void stage_tile_mixed(int* t3);
 
 } // namespace gr
