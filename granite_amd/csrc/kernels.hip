@@ -500,8 +500,8 @@ struct TileIODma {
 // The box is the packed one of the FP64 parts in floats, filled through registers one field ahead (the
 // deltas are formed on the way), by the pairs each lane would load directly: four 16-byte loads
 // and four 8-byte LDS writes a thread and field. 16x4x4 parts of 256 threads against whole 16x4x8
-// tiles of 512 with a box of single values and its corners (one workgroup per CU): two independent
-// workgroups per CU or, with the FP64 tiles beside them, one (128^3: stages 1-2 516 -> 485 us,
+// tiles of 512 with a box of single values and its corners: two or three independent workgroups per
+// CU instead of one (128^3: stages 1-2 516 -> 485 us,
 // stage 3 557 -> 521; 192^3 1665 -> 1551, 1800 -> 1673). At three waves per SIMD (168 registers) stage
 // 3 gains 2% at 128^3 and loses 7% at 101x77x59, where FP64 tiles are a larger share.
 // UN_IN: u^n is the stage input itself (the first stage, chosen at launch): its value at the
