@@ -122,12 +122,6 @@ __host__ __device__ GR_INLINE R tanh_(R x) {
     return tanh(x);
 }
 
-template <typename R>
-__host__ __device__ GR_INLINE R fma_(R a, R b, R c) {
-    using std::fma;
-    return fma(a, b, c);
-}
-
 // Forces x to be computed at this point of the instruction stream. Used on each field's
 // stencil results so that the compiler evaluates them before the next field is staged,
 // instead of keeping that field's raw neighbour values alive across later fields.
@@ -204,36 +198,6 @@ struct Advection {
     }
 };
 
-// 2nd-order mixed second derivatives
-template <typename R, class ST>
-__host__ __device__ GR_INLINE void mixed_derivs(const R* s, const Stencil<R>& K, const ST& st, R dd[6]) {
-    auto mixed = [&](int a, int b) {
-        return st.edge(s, a, b, 1, 1) - st.edge(s, a, b, 1, -1) - st.edge(s, a, b, -1, 1) + st.edge(s, a, b, -1, -1);
-    };
-    dd[1] = K.ihh[0] * mixed(0, 1);
-    dd[2] = K.ihh[1] * mixed(0, 2);
-    dd[4] = K.ihh[2] * mixed(1, 2);
-}
-
-// the results of a field are computed here, before the next field is staged
-template <bool D2, class ST, typename R>
-__host__ __device__ GR_INLINE void field_done(R d1[3], R dd[6], R& adv, R& ko) {
-#ifdef __HIP_DEVICE_COMPILE__
-    if constexpr (ST::READS_FIRST) {
-        __builtin_amdgcn_sched_group_barrier(0x100, 40, 0); // LDS reads
-        __builtin_amdgcn_sched_group_barrier(0x002, 400, 0); // then VALU
-    }
-#endif
-    pin(adv);
-    pin(ko);
-#pragma unroll
-    for (int d = 0; d < 3; ++d) pin(d1[d]);
-    if (D2) {
-#pragma unroll
-        for (int q = 0; q < 6; ++q) pin(dd[q]);
-    }
-}
-
 // All stencils of one field at one cell: 4th-order centred first derivative, one-sided
 // 5-point upwind derivative picked by the sign of beta (used only through the advection
 // sum), 7-point Kreiss-Oliger sum, and (D2) the 4th-order pure and 2nd-order mixed second
@@ -267,68 +231,29 @@ __host__ __device__ GR_INLINE void eval_field(const R* s, const Stencil<R>& K, c
             ko = (d == 0 ? R(0) : ko) + K.ko[d] * ((m3 + p3) - R(6) * (m2 + p2) + R(15) * (m1 + p1) - R(20) * c);
         if (D2) dd[sym(d, d)] = K.ih2[d] * (-p2 + R(16) * p1 - R(30) * c + R(16) * m1 - m2);
     }
-    if (D2) mixed_derivs(s, K, st, dd);
+    if (D2) {
+        auto mixed = [&](int a, int b) {
+            return st.edge(s, a, b, 1, 1) - st.edge(s, a, b, 1, -1) - st.edge(s, a, b, -1, 1) + st.edge(s, a, b, -1, -1);
+        };
+        dd[1] = K.ihh[0] * mixed(0, 1);
+        dd[2] = K.ihh[1] * mixed(0, 2);
+        dd[4] = K.ihh[2] * mixed(1, 2);
+    }
     if (!B.FOLDED) adv = B.w * upS + (R(1) - B.w) * cenS;
-    field_done<D2, ST>(d1, dd, adv, ko);
-}
-
-// Advection and dissipation of one field as one weighted sum of its taps, for the FP64 form and the
-// fields whose background value is zero (all but the metric, chi and the lapse, where the order
-// of the dissipation sum is kept: it decides the result where small structure lies on an O(1)
-// value). The weights of the cell, the same for all of these fields, hold both derivative
-// polynomials and the dissipation at the taps that all three read (the cell, one and two off);
-// the third and fourth taps are read on the upwind side only, and the dissipation's third ones
-// stay in `ko`, so that a tap enters no sum that it did not enter. 13 instructions per axis for 29;
-// 18 for A~ (KO_IN false), whose advection loses its trace and whose dissipation does not: there
-// the weights hold the advection alone.
-// Of the 4800 vector instructions of a wave 600 go (128^3: stages 1-2 483 -> 477 us, 101x77x59 130 ->
-// 125, a 96^3 right-hand side 206 -> 201): LDS reads and loads share the bound.
-// The fused operations are written out, so that every instance of the cell rounds alike.
-template <typename R>
-struct MergedTaps {
-    R c, p1[3], m1[3], p2[3], m2[3];
-    __host__ __device__ GR_INLINE void set(const Advection<R>& B, const Stencil<R>& K, bool ko_on) {
-#ifdef __clang__
-#pragma clang fp contract(off)
+#ifdef __HIP_DEVICE_COMPILE__
+    if constexpr (ST::READS_FIRST) {
+        __builtin_amdgcn_sched_group_barrier(0x100, 40, 0); // LDS reads
+        __builtin_amdgcn_sched_group_barrier(0x002, 400, 0); // then VALU
+    }
 #endif
-        c = R(0);
+    pin(adv);
+    pin(ko);
 #pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            const R k = ko_on ? K.ko[d] : R(0), u = B.up[d], e = B.cen[d] * K.ih[d];
-            const R ub = B.neg[d] ? u : R(0), uf = B.neg[d] ? R(0) : u;
-            c = fma_(R(-25), u, fma_(R(-20), k, c));
-            const R k1 = R(15) * k, k2 = R(-6) * k;
-            p1[d] = fma_(R(48), uf, fma_(R(8), e, k1));
-            m1[d] = fma_(R(48), ub, fma_(R(-8), e, k1));
-            p2[d] = fma_(R(-36), uf, k2 - e);
-            m2[d] = fma_(R(-36), ub, k2 + e);
-        }
-    }
-};
-
-// eval_field with the advection and (KO_IN) the dissipation's inner taps in `adv`
-template <bool D2, bool KO_IN, typename R, class ST>
-__host__ __device__ GR_INLINE void eval_merged(const R* s, const Stencil<R>& K, const ST& st, const Advection<R>& B,
-                                               const MergedTaps<R>& M, R d1[3], R dd[6], R& adv, R& ko) {
-    const R c = st.centre(s);
-    adv = M.c * c;
+    for (int d = 0; d < 3; ++d) pin(d1[d]);
+    if (D2) {
 #pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        const R m1 = st.at(s, d, -1), p1 = st.at(s, d, 1), m2 = st.at(s, d, -2), p2 = st.at(s, d, 2);
-        const R m3 = st.at(s, d, -3), p3 = st.at(s, d, 3), m4 = st.at(s, d, -4), p4 = st.at(s, d, 4);
-        d1[d] = K.ih[d] * (-p2 + R(8) * p1 - R(8) * m1 + m2);
-        adv = fma_(M.p1[d], p1, adv);
-        adv = fma_(M.m1[d], m1, adv);
-        adv = fma_(M.p2[d], p2, adv);
-        adv = fma_(M.m2[d], m2, adv);
-        adv = fma_(B.up[d], fma_(R(-3), B.side(d, m4, p4), R(16) * B.side(d, m3, p3)), adv);
-        R k = m3 + p3;
-        if (!KO_IN) k = fma_(R(-20), c, fma_(R(15), m1 + p1, fma_(R(-6), m2 + p2, k)));
-        ko = d == 0 ? K.ko[d] * k : fma_(K.ko[d], k, ko);
-        if (D2) dd[sym(d, d)] = K.ih2[d] * (-p2 + R(16) * p1 - R(30) * c + R(16) * m1 - m2);
+        for (int q = 0; q < 6; ++q) pin(dd[q]);
     }
-    if (D2) mixed_derivs(s, K, st, dd);
-    field_done<D2, ST>(d1, dd, adv, ko);
 }
 
 // Full RHS of one cell. `src` holds the matter sources at this cell when HAS_SRC.
@@ -377,9 +302,6 @@ __host__ __device__ GR_INLINE void ccz4_cell(Stager& S, Sink& O, const Stencil<R
     B.set(be, R(0.5) * (R(1) + tanh_((chi - R(P.chi_c)) / R(P.chi_w))), K.ih);
 
     R d1[3], dd[6], adv, ko;
-    constexpr bool MERGED = Advection<R>::FOLDED;
-    MergedTaps<R> M;
-    if constexpr (MERGED) M.set(B, K, O.ko_on);
 
     // Gamma-hat RHS (ccz4.cpp:747-815) is gathered in GA as its ingredients appear:
     // T5 + T6 from the shift's second derivatives, T1 + T4 + T8 once the Christoffels and
@@ -391,10 +313,7 @@ __host__ __device__ GR_INLINE void ccz4_cell(Stager& S, Sink& O, const Stencil<R
     R dbe[3][3], ddiv[3] = {R(0), R(0), R(0)};
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
-        if constexpr (MERGED)
-            eval_merged<true, true>(S.field(BX + c), K, S.strides(), B, M, d1, dd, adv, ko);
-        else
-            eval_field<true, KO_EXACT>(S.field(BX + c), K, S.strides(), B, d1, dd, adv, ko);
+        eval_field<true, KO_EXACT>(S.field(BX + c), K, S.strides(), B, d1, dd, adv, ko);
         R t5 = R(0);
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
@@ -579,24 +498,9 @@ __host__ __device__ GR_INLINE void ccz4_cell(Stager& S, Sink& O, const Stencil<R
     for (int p = 0; p < 6; ++p) pin(Rt[p]);
 
     // ---- K (ccz4.cpp:621-652); its gradient completes T2 of Gamma-hat
-    // the weights are formed again rather than kept live across the metric's derivatives
-    if constexpr (MERGED) {
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            pin(B.up[d]);
-            pin(B.cen[d]);
-        }
-        M.set(B, K, O.ko_on);
-    }
-    auto small_field = [&](int v, R der[3], R& ad, R& dis) {
-        if constexpr (MERGED)
-            eval_merged<false, true>(S.field(v), K, S.strides(), B, M, der, dd, ad, dis);
-        else
-            eval_field<false, KO_EXACT>(S.field(v), K, S.strides(), B, der, dd, ad, dis);
-    };
     {
         R dK[3];
-        small_field(KTR, dK, adv, ko);
+        eval_field<false, KO_EXACT>(S.field(KTR), K, S.strides(), B, dK, dd, adv, ko);
         const R matter = HAS_SRC ? R(4) * R(PI) * alpha * (R(src.rho) + R(src.S)) : R(0);
         O.put(KTR,
               -plap + alpha * (AA + Ktr * Ktr / R(3)) + matter + R(P.kappa1) * (R(1) - R(P.kappa2)) * alpha * Theta + adv,
@@ -617,7 +521,7 @@ __host__ __device__ GR_INLINE void ccz4_cell(Stager& S, Sink& O, const Stencil<R
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
         R advq, koq;
-        small_field(GHX + q, d1, advq, koq);
+        eval_field<false, KO_EXACT>(S.field(GHX + q), K, S.strides(), B, d1, dd, advq, koq);
 #pragma unroll
         for (int p = 0; p < 6; ++p) {
             const int a = sym_a(p), b = sym_b(p);
@@ -640,7 +544,7 @@ __host__ __device__ GR_INLINE void ccz4_cell(Stager& S, Sink& O, const Stencil<R
     pin(Rs);
 
     // ---- Theta (ccz4.cpp:654-665)
-    small_field(THETA, d1, adv, ko);
+    eval_field<false, KO_EXACT>(S.field(THETA), K, S.strides(), B, d1, dd, adv, ko);
     {
         const R rho = HAS_SRC ? R(src.rho) : R(0);
         O.put(THETA,
@@ -651,14 +555,10 @@ __host__ __device__ GR_INLINE void ccz4_cell(Stager& S, Sink& O, const Stencil<R
 
     // ---- A~: raw value, then trace removed with the full raw trace (ccz4.cpp:671-726)
     R raw[6], koA[6];
-    if constexpr (MERGED) M.set(B, K, false);
 #pragma unroll
     for (int p = 0; p < 6; ++p) {
         const int a = sym_a(p), b = sym_b(p);
-        if constexpr (MERGED)
-            eval_merged<false, false>(S.field(AXX + p), K, S.strides(), B, M, d1, dd, adv, koA[p]);
-        else
-            eval_field<false, KO_EXACT>(S.field(AXX + p), K, S.strides(), B, d1, dd, adv, koA[p]);
+        eval_field<false, KO_EXACT>(S.field(AXX + p), K, S.strides(), B, d1, dd, adv, koA[p]);
         const R t1 = HAS_SRC ? chi * (XA[p] - alpha * R(8) * R(PI) * R(src.Sij[p])) : chi * XA[p];
         R Aub[3]; // A^q_b = g^qr A_rb
 #pragma unroll
