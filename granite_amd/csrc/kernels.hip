@@ -945,12 +945,16 @@ __device__ __forceinline__ double f_inf(int v) {
     return (v == 0 || v == 1 || v == 4 || v == 6 || v == 18) ? 1.0 : 0.0;
 }
 
-// a / b from inv = 1 / b, correctly rounded: the quotient, its exact remainder and one correction
-// (Markstein's theorem), with the hardware's rule for zeros, infinities and NaN. Four instructions
-// where a division by itself takes eleven.
+// a / b from inv = 1 / b, correctly rounded unless tiny_quotient(a, b): the quotient, its exact remainder
+// and one correction (Markstein's theorem), with the hardware's rule for zeros, infinities and NaN. Four
+// instructions where a division by itself takes eleven.
 __device__ __forceinline__ double quotient(double a, double b, double inv) {
     const double q = a * inv;
     return __builtin_amdgcn_div_fixup(fma(fma(-q, b, a), inv, q), b, a);
+}
+// whether a / b may be subnormal (rounded twice above) or its remainder inexact
+__device__ __forceinline__ bool tiny_quotient(double a, double b) {
+    return (fabs(a) < 0x1p-900 && a != 0.0) || b > 0x1p100;
 }
 
 // Final value of a ghost cell after the reference's three passes: each pass over axis d
@@ -1032,12 +1036,13 @@ __device__ void fill_ghost_cell(const BlockDesc& b, gdouble* u, long t_, int mod
 #pragma unroll
     for (int m = 0; m < NF; ++m) {
         const int v = g + G * m;
-        if (v < NV) val[m] = u[v * b.stride + src];
+        val[m] = v < NV ? u[v * b.stride + src] : 0.0;
     }
     if (mode == 0) {
         // (r_int, r_gh) of each step of the chain: start at the anchor, move one ghost axis
         // at a time in X, Y, Z order
         double Q[3] = {coord(b, 0, A[0]), coord(b, 1, A[1]), coord(b, 2, A[2])};
+        bool tiny = false;
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
             if (!gh[d]) continue;
@@ -1047,9 +1052,28 @@ __device__ void fill_ghost_cell(const BlockDesc& b, gdouble* u, long t_, int mod
             const double inv = 1.0 / rgh;
 #pragma unroll
             for (int m = 0; m < NF; ++m) {
-                const double fi = f_inf(g + G * m);
-                val[m] = fi + quotient((val[m] - fi) * rin, rgh, inv);
+                const double fi = f_inf(g + G * m), a = (val[m] - fi) * rin;
+                tiny = tiny || tiny_quotient(a, rgh);
+                val[m] = fi + quotient(a, rgh, inv);
             }
+        }
+        // once more by divisions (same launch: the anchor still holds its value)
+        if (tiny) {
+#pragma unroll 1
+            for (int v = g; v < NV; v += G) {
+                const double fi = f_inf(v);
+                double x = u[v * b.stride + src];
+                double P[3] = {coord(b, 0, A[0]), coord(b, 1, A[1]), coord(b, 2, A[2])};
+#pragma unroll
+                for (int d = 0; d < 3; ++d) {
+                    if (!gh[d]) continue;
+                    const double rin = radius(P[0], P[1], P[2]);
+                    P[d] = coord(b, d, I[d]);
+                    x = fi + ((x - fi) * rin) / radius(P[0], P[1], P[2]);
+                }
+                u[v * b.stride + dst] = x;
+            }
+            return;
         }
     }
 #pragma unroll
@@ -1264,8 +1288,9 @@ __global__ __launch_bounds__(GHOST_WG) void fill_ghosts_batch_kernel(const Batch
                                          int sel, int mode) {
     const BatchBlock& B = table[wg_block[blockIdx.x]]; // one block per workgroup
     const long t = (long)(blockIdx.x - B.ghost_wg0) * GHOST_WG + threadIdx.x;
-    if (t >= ghost_count(B.b)) return;
-    fill_ghost_cell<G>(B.b, (gdouble*)B.buf[sel], t, mode, 0x3f, blockIdx.y);
+    const BlockDesc b = B.b; // (not read again behind the stores)
+    if (t >= ghost_count(b)) return;
+    fill_ghost_cell<G>(b, (gdouble*)B.buf[sel], t, mode, 0x3f, blockIdx.y);
 }
 
 // ------------------------------------------------------------------------------------
