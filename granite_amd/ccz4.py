@@ -325,6 +325,8 @@ class Engine:
             raise EngineError(rc, f"no usable gfx950 device {device}")
         self._h = h
         self.lib = L
+        self._users = set()  # objects that hold native parts of this engine
+        self._parting = None  # closed, to be destroyed after the last of them
 
     @classmethod
     def default(cls) -> "Engine":
@@ -344,9 +346,17 @@ class Engine:
         self.check(self.lib.gr_engine_sync(self._h))
 
     def close(self):
-        if self._h:
-            self.lib.gr_engine_destroy(self._h)
-            self._h = None
+        """Closes the engine; its native part outlives the levels, hierarchies and checkpoints made
+        from it (the garbage collector finalises a cycle of them in any order)."""
+        h, self._h = self._h, None
+        self._parting = self._parting or h
+        self._release(None)
+
+    def _release(self, user):
+        self._users.discard(user)
+        if self._parting and not self._users:
+            h, self._parting = self._parting, None
+            self.lib.gr_engine_destroy(h)
 
     def __del__(self):
         try:
@@ -411,6 +421,7 @@ class Level:
         h = C.c_void_p()
         self._e.check(self._e.lib.gr_level_create(self._e.handle, len(self.blocks), geoms, C.byref(h)))
         self._h = h
+        self._e._users.add(id(self))
 
     def upload(self, i=None):
         for b in range(len(self.blocks)) if i is None else [i]:
@@ -532,6 +543,7 @@ class Level:
         if getattr(self, "_h", None):
             self._e.lib.gr_level_destroy(self._h)
             self._h = None
+            self._e._release(id(self))
 
     def __del__(self):
         try:
@@ -554,6 +566,7 @@ class Hierarchy:
         h = C.c_void_p()
         self._e.check(self._e.lib.gr_hierarchy_create(self._e.handle, len(self.levels), arr, C.byref(h)))
         self._h = h
+        self._e._users.add(id(self))
 
     def prolongate(self, level):
         self._e.check(self._e.lib.gr_hierarchy_prolongate(self._h, int(level)))
@@ -612,6 +625,7 @@ class Hierarchy:
         if getattr(self, "_h", None):
             self._e.lib.gr_hierarchy_destroy(self._h)
             self._h = None
+            self._e._release(id(self))
 
     def __del__(self):
         try:
@@ -633,6 +647,7 @@ class Checkpoint:
         h = C.c_void_p()
         self._e.check(self._e.lib.gr_checkpoint_create(self._e.handle, len(self.levels), arr, C.byref(h)))
         self._h = h
+        self._e._users.add(id(self))
         self._geoms = [(lv, b) for lv in self.levels for b in lv.blocks]
 
     def begin(self):
@@ -664,6 +679,7 @@ class Checkpoint:
         if getattr(self, "_h", None):
             self._e.lib.gr_checkpoint_destroy(self._h)
             self._h = None
+            self._e._release(id(self))
 
     def __del__(self):
         try:
