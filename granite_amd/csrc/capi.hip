@@ -47,12 +47,18 @@ struct gr_engine {
     gr::AuxStream aux{nullptr, nullptr, nullptr}; // runs the FP64 tiles beside the FP32 ones
     std::string err;
     // multi-level step: a second stream for the ghost fills, events ordering each level's
-    // stages and fills, and the captured graph of the last level set
+    // stages and fills, and the captured graphs of the level sets
     hipStream_t fill_stream = nullptr;
     std::vector<hipEvent_t> ls_events;
-    hipGraph_t ls_graph = nullptr;
-    hipGraphExec_t ls_exec = nullptr;
-    std::vector<double> ls_key;
+    struct {
+        hipGraph_t graph = nullptr;
+        hipGraphExec_t exec = nullptr;
+        std::vector<double> key;
+    } ls[2]; // by precision
+    // a captured step that was let go of, held until its last launch has ended (drop_graph)
+    hipGraph_t dropped_graph = nullptr;
+    hipGraphExec_t dropped_exec = nullptr;
+    hipEvent_t dropped_end = nullptr;
     // compatibility-mode staging buffers (grown on demand, doubles)
     double* d_u = nullptr;
     double* d_r = nullptr;
@@ -214,6 +220,16 @@ int gr_stage_tile(int precision, int* t3) {
     return GR_OK;
 }
 
+// the captured step let go of before (drop_graph), whose last launch has ended
+static hipError_t free_dropped(gr_engine* e) {
+    hipError_t st = hipSuccess;
+    if (e->dropped_exec) st = hipGraphExecDestroy(e->dropped_exec);
+    e->dropped_exec = nullptr;
+    const hipError_t st2 = e->dropped_graph ? hipGraphDestroy(e->dropped_graph) : hipSuccess;
+    e->dropped_graph = nullptr;
+    return st != hipSuccess ? st : st2;
+}
+
 int gr_engine_create(int device, gr_engine** out) {
     if (!out) return GR_ERR_ARG;
     *out = nullptr;
@@ -259,8 +275,12 @@ int gr_engine_destroy(gr_engine* e) {
     if (e->aux.fork) (void)hipEventDestroy(e->aux.fork);
     if (e->aux.join) (void)hipEventDestroy(e->aux.join);
     if (e->aux.stream) (void)hipStreamDestroy(e->aux.stream);
-    if (e->ls_exec) (void)hipGraphExecDestroy(e->ls_exec);
-    if (e->ls_graph) (void)hipGraphDestroy(e->ls_graph);
+    for (auto& ls : e->ls) {
+        if (ls.exec) (void)hipGraphExecDestroy(ls.exec);
+        if (ls.graph) (void)hipGraphDestroy(ls.graph);
+    }
+    (void)free_dropped(e);
+    if (e->dropped_end) (void)hipEventDestroy(e->dropped_end);
     for (hipEvent_t ev : e->ls_events) (void)hipEventDestroy(ev);
     if (e->fill_stream) {
         (void)hipStreamSynchronize(e->fill_stream);
@@ -729,11 +749,13 @@ int gr_level_destroy(gr_level* L) {
         (void)hipStreamSynchronize(e->stream);
         if (e->fill_stream) (void)hipStreamSynchronize(e->fill_stream);
         // a captured level-set step may hold this level's buffers
-        if (e->ls_exec) (void)hipGraphExecDestroy(e->ls_exec);
-        if (e->ls_graph) (void)hipGraphDestroy(e->ls_graph);
-        e->ls_exec = nullptr;
-        e->ls_graph = nullptr;
-        e->ls_key.clear();
+        for (auto& ls : e->ls) {
+            if (ls.exec) (void)hipGraphExecDestroy(ls.exec);
+            if (ls.graph) (void)hipGraphDestroy(ls.graph);
+            ls.exec = nullptr;
+            ls.graph = nullptr;
+            ls.key.clear();
+        }
     }
     if (L->exec) (void)hipGraphExecDestroy(L->exec);
     if (L->graph) (void)hipGraphDestroy(L->graph);
@@ -947,6 +969,24 @@ static hipError_t enqueue_levels_rk3(gr_engine* e, int n, gr_level* const* lv, c
     return st;
 }
 
+// Lets go of a captured step. Its last launch may still be running, and the runtime does not promise to
+// keep what a running launch uses, so the engine holds the graph until that launch has ended: at the
+// next call here, which waits for it. One is held at a time, and a new capture still overlaps the
+// step before it (a step captured anew on every call: 64^3 229 us, with a wait for the stream 306).
+static hipError_t drop_graph(gr_engine* e, hipGraph_t* graph, hipGraphExec_t* exec) {
+    if (!*exec && !*graph) return hipSuccess;
+    hipError_t st = hipSuccess;
+    if (!e->dropped_end) st = hipEventCreateWithFlags(&e->dropped_end, hipEventDisableTiming);
+    if (st == hipSuccess && e->dropped_exec) st = hipEventSynchronize(e->dropped_end);
+    if (st == hipSuccess) st = free_dropped(e);
+    if (st != hipSuccess) return st;
+    e->dropped_graph = *graph;
+    e->dropped_exec = *exec;
+    *graph = nullptr;
+    *exec = nullptr;
+    return hipEventRecord(e->dropped_end, e->stream);
+}
+
 extern "C" {
 
 int gr_level_rk3_step(gr_level* L, const gr_ccz4_params* prm, double dt, int precision, int bc_mode, int pre_fill,
@@ -968,11 +1008,8 @@ int gr_level_rk3_step(gr_level* L, const gr_ccz4_params* prm, double dt, int pre
                             prm->chi_blend_width, (double)precision, (double)bc_mode, (double)pre_fill,
                             (double)L->generation};
     if (!L->have_graph || std::memcmp(key, L->gkey, sizeof(key)) != 0) {
-        if (L->exec) GR_HIP(e, hipGraphExecDestroy(L->exec));
-        if (L->graph) GR_HIP(e, hipGraphDestroy(L->graph));
-        L->exec = nullptr;
-        L->graph = nullptr;
         L->have_graph = false;
+        GR_HIP(e, drop_graph(e, &L->graph, &L->exec));
         GR_HIP(e, hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal));
         hipError_t st = enqueue_rk3(L, prm, dt, bc_mode, pre_fill, precision);
         hipGraph_t g = nullptr;
@@ -1020,12 +1057,10 @@ int gr_levels_rk3_step(int n, gr_level* const* levels, const double* dts, const 
         key.push_back((double)levels[i]->generation);
         key.push_back(dts[i]);
     }
-    if (!e->ls_exec || key != e->ls_key) {
-        if (e->ls_exec) GR_HIP(e, hipGraphExecDestroy(e->ls_exec));
-        if (e->ls_graph) GR_HIP(e, hipGraphDestroy(e->ls_graph));
-        e->ls_exec = nullptr;
-        e->ls_graph = nullptr;
-        e->ls_key.clear();
+    auto& ls = e->ls[precision == GR_PREC_MIXED ? 1 : 0];
+    if (!ls.exec || key != ls.key) {
+        ls.key.clear();
+        GR_HIP(e, drop_graph(e, &ls.graph, &ls.exec));
         GR_HIP(e, hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal));
         hipError_t st = enqueue_levels_rk3(e, n, levels, dts, prm, bc_mode, pre_fill, precision);
         hipGraph_t g = nullptr;
@@ -1035,11 +1070,11 @@ int gr_levels_rk3_step(int n, gr_level* const* levels, const double* dts, const 
             return hipfail(e, st, "capture of the level-set step");
         }
         if (st2 != hipSuccess) return hipfail(e, st2, "hipStreamEndCapture");
-        e->ls_graph = g;
-        GR_HIP(e, hipGraphInstantiate(&e->ls_exec, e->ls_graph, nullptr, nullptr, 0));
-        e->ls_key = key;
+        ls.graph = g;
+        GR_HIP(e, hipGraphInstantiate(&ls.exec, ls.graph, nullptr, nullptr, 0));
+        ls.key = key;
     }
-    GR_HIP(e, hipGraphLaunch(e->ls_exec, e->stream));
+    GR_HIP(e, hipGraphLaunch(ls.exec, e->stream));
     return GR_OK;
 }
 
@@ -1763,11 +1798,8 @@ int gr_hierarchy_step(gr_hierarchy* H, const gr_ccz4_params* prm, double dt0, in
     policy.push_back(H->cfl_on ? 1.0 : 0.0);
     const bool fresh = H->have_graph && std::memcmp(key, H->gkey, sizeof(key)) == 0 && policy == H->policy;
     if (!fresh) {
-        if (H->exec) GR_HIP(e, hipGraphExecDestroy(H->exec));
-        if (H->graph) GR_HIP(e, hipGraphDestroy(H->graph));
-        H->exec = nullptr;
-        H->graph = nullptr;
         H->have_graph = false;
+        GR_HIP(e, drop_graph(e, &H->graph, &H->exec));
         GR_HIP(e, hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal));
         hipError_t st = h_step(H, dt0, prm, precision);
         hipGraph_t g = nullptr;
