@@ -1058,6 +1058,12 @@ int gr_levels_rk3_step(int n, gr_level* const* levels, const double* dts, const 
         key.push_back(dts[i]);
     }
     auto& ls = e->ls[precision == GR_PREC_MIXED ? 1 : 0];
+    if (ls.exec && key != ls.key && precision == GR_PREC_MIXED) {
+        // Capturing a mixed level set while the graph of another one is held has ended the process in
+        // the runtime, for a cause not known: such a call runs eager, with the same results.
+        GR_HIP(e, enqueue_levels_rk3(e, n, levels, dts, prm, bc_mode, pre_fill, precision));
+        return GR_OK;
+    }
     if (!ls.exec || key != ls.key) {
         ls.key.clear();
         GR_HIP(e, drop_graph(e, &ls.graph, &ls.exec));

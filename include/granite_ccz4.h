@@ -181,7 +181,8 @@ int gr_level_set_mixed_policy(gr_level* lvl, double chi_fp64_below);
  * (compute-bound); each level's own stages and fills keep their order (events). Results are
  * bit-identical to stepping the levels one by one. use_graph: the whole schedule as one
  * captured HIP graph, re-captured when the level set, a dt, the parameters or a level's
- * tuning change. */
+ * tuning change; in the mixed form only the first level set, until one of the engine's levels is
+ * destroyed: calls with another key run the same launches eager. */
 int gr_levels_rk3_step(int n, gr_level* const* levels, const double* dts, const gr_ccz4_params* prm, int precision,
                        int bc_mode, int pre_fill, int use_graph);
 

@@ -33,7 +33,7 @@ def same(a, b):
         lb.close()
 
 
-@pytest.mark.parametrize("precision", [0])
+@pytest.mark.parametrize("precision", [0, 1])
 def test_alternating_level_sets(engine, precision):
     import granite_amd as ga
 
