@@ -601,6 +601,12 @@ void tune_put(int kind, int cls, int prec, int v) {
     g_tune[std::make_tuple(kind, cls, prec)] = v;
 }
 
+// First line of a saved table. Tables of earlier builds name stagings of the stage kernel that are gone:
+// their values 1 and 2 would now force a part shape, so their stage entries are not taken and those
+// classes keep the default.
+constexpr const char* kTuneHeader = "# granite-ccz4 tuning table, stage forms by part shape: kind class precision value";
+constexpr const char* kTuneHeaderOld = "# granite-ccz4 tuning table: kind class precision value";
+
 bool tune_valid(int kind, int v) {
     if (kind == GR_TUNE_STAGE) return v >= 0 && v < gr::FP64_STAGE_VARIANTS;
     return gr::ghost_groups_valid(v); // GR_TUNE_GHOST, GR_TUNE_TRANSFER
@@ -1486,7 +1492,7 @@ int gr_tune_save(const char* path) {
     std::ofstream f(path);
     if (!f) return GR_ERR_ARG;
     std::lock_guard<std::mutex> lock(g_tune_mu);
-    f << "# granite-ccz4 tuning table: kind class precision value\n";
+    f << kTuneHeader << '\n';
     for (const auto& kv : g_tune)
         f << std::get<0>(kv.first) << ' ' << std::get<1>(kv.first) << ' ' << std::get<2>(kv.first) << ' ' << kv.second
           << '\n';
@@ -1499,8 +1505,10 @@ int gr_tune_load(const char* path) {
     if (!f) return GR_ERR_ARG;
     std::vector<std::pair<std::tuple<int, int, int>, int>> rows;
     std::string line;
+    bool old_forms = false;
     while (std::getline(f, line)) {
         const size_t p = line.find_first_not_of(" \t\r");
+        if (p != std::string::npos && line.compare(p, std::strlen(kTuneHeaderOld), kTuneHeaderOld) == 0) old_forms = true;
         if (p == std::string::npos || line[p] == '#') continue;
         std::istringstream in(line);
         int kind = -1, cls = -1, prec = -1, value = -1;
@@ -1509,6 +1517,7 @@ int gr_tune_load(const char* path) {
         if (kind < GR_TUNE_STAGE || kind > GR_TUNE_TRANSFER || cls < 0 || cls > 3 || prec < 0 || prec > 1 ||
             !tune_valid(kind, value))
             return GR_ERR_ARG;
+        if (old_forms && kind == GR_TUNE_STAGE) continue;
         rows.push_back({std::make_tuple(kind, cls, prec), value});
     }
     std::lock_guard<std::mutex> lock(g_tune_mu);
