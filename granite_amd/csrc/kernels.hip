@@ -1909,10 +1909,12 @@ Batch single_batch(const BlockDesc& b, const double* in, const double* un, doubl
     return B;
 }
 
+bool stage_parts_large(const Batch& B) { return B.variant == 2 || (B.variant == 0 && B.ntiles >= LARGE_TILES); }
+
 hipError_t launch_stage_fp64(const Batch& B, const int sel[3], bool has_src, const CellParams& P,
                              double ko_sigma, int mode, const StageCoef& cf, hipStream_t s,
                              const unsigned char* flags) {
-    const bool large = B.variant == 2 || (B.variant == 0 && B.ntiles >= LARGE_TILES);
+    const bool large = stage_parts_large(B);
     StageArgs A = stage_args(B, sel, P, ko_sigma, cf, flags, 1);
     // with flags (the FP64 tiles of the mixed form: few, near the puncture) a small grid
     // gathers them instead of launching one workgroup per part of every tile of the level

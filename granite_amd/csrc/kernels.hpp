@@ -68,6 +68,8 @@ struct Batch {
     int variant;  // FP64 form of the stage kernel
     int ghost_groups; // field groups of the ghost fill launch (1, 2, 4 or 11)
 };
+// whether an FP64 stage launch of B runs the large parts (16x4x4), by its form or its size
+bool stage_parts_large(const Batch& B);
 // whether block b's rows can be read as aligned 16-byte pairs from buffer p
 bool pairs_aligned(const BlockDesc& b, const void* p);
 
