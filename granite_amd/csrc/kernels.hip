@@ -1909,7 +1909,10 @@ Batch single_batch(const BlockDesc& b, const double* in, const double* un, doubl
     return B;
 }
 
-bool stage_parts_large(const Batch& B) { return B.variant == 2 || (B.variant == 0 && B.ntiles >= LARGE_TILES); }
+bool stage_parts_large(const Batch& B) {
+    const int form = B.pairs_ok ? B.variant : 0;
+    return form == 2 || (form == 0 && B.ntiles >= LARGE_TILES);
+}
 
 hipError_t launch_stage_fp64(const Batch& B, const int sel[3], bool has_src, const CellParams& P,
                              double ko_sigma, int mode, const StageCoef& cf, hipStream_t s,
