@@ -9,6 +9,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <sched.h>
+
 #include <algorithm>
 #include <array>
 #include <atomic>
@@ -306,24 +308,37 @@ namespace {
 
 // The host call of the right-hand side moves the state in and the interior of the result out,
 // through pinned memory that several threads fill and empty beside the copies; the caller's
-// ghost cells of the result are not touched, so they are not sent either.
-// Three direct copies of pageable memory (state in, result in for its ghosts, result out) against
-// this, us: 12^3 223 -> 126, 24^3 697 -> 330, 48^3 3940 -> 1545, 80^3 15300 -> 5200. Pinned memory
-// is bounded; a block above the bound (90^3 and more) keeps the direct copies, as does memory
-// that the host cannot read by itself.
+// ghost cells of the result are not touched, so they are not sent either. A state that is pinned
+// already is sent as it is.
+// Three direct copies (state in, result in for its ghosts, result out) against this, us: pageable
+// arrays 12^3 220 -> 125, 24^3 700 -> 330, 48^3 3800 -> 1540, 80^3 15000 -> 5200, on a single CPU 80^3 15000 ->
+// 10000; pinned arrays 12^3 130 -> 97, 32^3 650 -> 550 (staged 770), 48^3 1706 -> 1320, 80^3 6510 -> 4800.
+// Pinned memory is bounded: a block above the bound (from 84^3 on) keeps the direct copies, as does
+// memory that the host cannot read by itself, and a pinned result of a process with one CPU, which
+// empties the staging more slowly than the bus would carry the result (56^3 2590 against 2540, 80^3 7840
+// against 6510; 48^3 1520 against 1706).
 constexpr size_t kStageMaxBytes = 128u << 20;     // larger blocks keep the direct copies
+constexpr size_t kStageMaxBytesOneCpu = 40u << 20; // .. and these, of a pinned result and one CPU
 constexpr size_t kStageBytesPerThread = 4u << 20; // a thread more per 4 MiB of state ..
 constexpr int kStageMaxThreads = 8;               // .. up to 8
 constexpr int kStageChunks = 11;                  // of two fields each with several threads, else one
 
-// whether p is memory the host can copy by itself (not device memory)
-bool host_readable(const void* p) {
+// whether p is memory the host can copy by itself (not device memory), and whether it is pinned
+bool host_readable(const void* p, bool* pinned) {
     hipPointerAttribute_t a;
+    *pinned = false;
     if (hipPointerGetAttributes(&a, p) != hipSuccess) {
         (void)hipGetLastError(); // not known to the runtime: ordinary host memory
         return true;
     }
+    *pinned = a.type == hipMemoryTypeHost;
     return a.type == hipMemoryTypeHost || a.type == hipMemoryTypeUnregistered;
+}
+
+// CPUs this thread may run on
+int usable_cpus() {
+    cpu_set_t set;
+    return sched_getaffinity(0, sizeof(set), &set) == 0 ? CPU_COUNT(&set) : (int)std::thread::hardware_concurrency();
 }
 
 // pinned staging for n doubles and the chunks' events; false: not to be had, use direct copies
@@ -355,6 +370,7 @@ struct StagedRhs {
     const gr::BlockDesc& b;
     const double* u;
     double* rhs;
+    bool u_pinned; // u needs no staging
     std::atomic<int> in{0}, out{0};       // next field to send, next chunk to scatter
     std::atomic<int> status{hipSuccess};  // first error of any thread
     std::mutex m;
@@ -392,7 +408,7 @@ struct StagedRhs {
     }
     void help() {
         note(hipSetDevice(e->device));
-        send();
+        if (!u_pinned) send();
         {
             std::unique_lock<std::mutex> l(m);
             ++sent;
@@ -412,7 +428,7 @@ struct StagedRhs {
             for (; helpers + 1 < want; ++helpers) t[helpers] = std::thread([this] { help(); });
         } catch (...) { // no thread to be had: the calling one does the rest
         }
-        if (helpers)
+        if (helpers && !u_pinned)
             send();
         else
             note(hipMemcpyAsync(e->d_u, u, bytes, hipMemcpyHostToDevice, e->stream));
@@ -475,8 +491,10 @@ int gr_ccz4_rhs(gr_engine* e, const gr_geom* geom, const gr_ccz4_params* prm, in
                                      cell_params(prm), prm->ko_sigma, gr::MODE_RHS, gr::StageCoef{0.0, 0.0, 0.0},
                                      e->stream);
     };
-    if (host_readable(u) && host_readable(rhs) && stage_ready(e, n)) {
-        StagedRhs call{e, b, u, rhs};
+    bool u_pinned = false, rhs_pinned = false;
+    if (host_readable(u, &u_pinned) && host_readable(rhs, &rhs_pinned) &&
+        !(rhs_pinned && n * sizeof(double) > kStageMaxBytesOneCpu && usable_cpus() == 1) && stage_ready(e, n)) {
+        StagedRhs call{e, b, u, rhs, u_pinned};
         GR_HIP(e, call.run(launch));
         return GR_OK;
     }
