@@ -743,8 +743,8 @@ int gr_level_create(gr_engine* e, int nblocks, const gr_geom* geoms, gr_level** 
         if (st != hipSuccess) break;
         st = build_batch(L, G.blocks, G.table, &G.d_table, &G.d_tile_block, &G.d_ghost_wg_block, &G.batch);
         if (st == hipSuccess) st = hipMalloc((void**)&G.flags, G.batch.ntiles);
-        // without a table entry: the large parts where the rows allow forcing them and the launch is
-        // large enough to fill the machine (at least 40^3 cells), else the launch's own choice
+        // without a table entry: form 2 from 40^3 cells on where the rows allow it, else the launch's own
+        // choice (which from 40^3 cells on, 125 tiles, is the same kernel)
         double cells = 0.0;
         for (int i : G.blocks) cells += (double)L->blk[i].n[0] * L->blk[i].n[1] * L->blk[i].n[2];
         int v = (G.batch.pairs_ok && cells >= 40.0 * 40 * 40) ? 2 : 0;

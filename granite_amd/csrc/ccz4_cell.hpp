@@ -76,25 +76,12 @@ struct Stencil {
     R kw[3][4];
 };
 
-// Index strides of a staged array along x, y, z. The LDS tile uses compile-time strides
-// so that every stencil tap is an immediate offset from one base address. READS_FIRST asks the
-// compiler to issue a field's reads ahead of its arithmetic (eval_field).
-template <int SX, int SY, int SZ>
-struct FixedStrides {
-    static constexpr bool READS_FIRST = false;
-    __host__ __device__ static constexpr long q(int d) { return d == 0 ? SX : (d == 1 ? SY : SZ); }
-    // value at the cell, k cells off along axis d, and i cells off along a and j along b
-    template <typename R>
-    __host__ __device__ static R centre(const R* s) { return s[0]; }
-    template <typename R>
-    __host__ __device__ static R at(const R* s, int d, int k) { return s[k * q(d)]; }
-    template <typename R>
-    __host__ __device__ static R edge(const R* s, int a, int b, int i, int j) { return s[i * q(a) + j * q(b)]; }
-};
+// Taps of a field stored as a whole array: the value at the cell, k cells off along axis d, and i
+// cells off along a and j along b, by index strides. (The staged fields have taps of their own.)
+// READS_FIRST asks the compiler to issue a field's reads ahead of its arithmetic (eval_field).
 struct RuntimeStrides {
     static constexpr bool READS_FIRST = false;
     long s[3];
-    __host__ __device__ long q(int d) const { return s[d]; }
     template <typename R>
     __host__ __device__ static R centre(const R* p) { return p[0]; }
     template <typename R>
@@ -174,7 +161,7 @@ struct Advection {
         return r;
     }
     // the FP32 form's code is scheduled better with the compiler's own selects and the blend at the
-    // end (measured on a 128^3 stage: 505 us against 580)
+    // end (128^3 stages 1-2, whole tiles of 512 threads as it was then: 505 us against 580)
     __device__ __forceinline__ float side(int d, float b, float f) const { return neg[d] ? b : f; }
     __device__ __forceinline__ double side(int d, double b, double f) const {
         const unsigned lo = move(back[d], (unsigned)__double2loint(b), (unsigned)__double2loint(f));

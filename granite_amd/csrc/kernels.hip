@@ -141,10 +141,11 @@ constexpr bool lds_conflict_free(int P, int Q) {
 // -2, TZ + 1 .. TZ + 3) only the z axis reads the part's own 16 x 4 columns: their rows go, two to a block
 // of 32 doubles, into the hole of the lower outer plane (A) and after the end (TE: even rows, TO:
 // odd rows), each at the place modulo 32 doubles it would have in a plane of its own, so that the
-// z taps stay free of bank conflicts. Parts of 16 x 4 x 4 take 16 KiB a field (a whole box 27) and, with the
-// rows 64-byte aligned, 158 cache lines (8 x 4 x 8 parts of the same size: 188): lines fetched into
-// the CU, not bytes from memory or arithmetic, are what a stage costs most (128^3, stages 1-2: 8x4x8
-// whole boxes 570 us, packed 535, 16x4x4 packed 508).
+// z taps stay free of bank conflicts. Parts of 16 x 4 x 4 take 16 KiB
+// a field (a whole box 27) and, with the rows 64-byte aligned, 158 cache lines (8 x 4 x 8 parts of the
+// same size: 188). 128^3, stages 1-2: 8x4x8 whole boxes 570 us, packed 535, 16x4x4 packed 508. Lines are one
+// cost among several: the kernel without its loads took 75 us less, without its stores 92, without its
+// LDS reads 87, and 16x4x8 parts, with a fifth fewer lines a cell, gained nothing.
 template <int TZ>
 struct PackedBox {
     static constexpr int TX = 16, TY = 4;
@@ -973,10 +974,10 @@ __device__ __forceinline__ long ghost_count(const BlockDesc& b) {
 // (src/amr/amr.cpp:412-480).
 // Fields g, g + G, ... of the cell: the G field groups run as separate workgroups (second
 // grid dimension), so a small ghost region still fills the machine.
-// Bound by memory: at 192^3 91 us for 290 MB read and 159 MB written, 4.9 TB/s, 56 us of them (6 of
+// Bound by memory: at 192^3 92 us for 290 MB read and 159 MB written, 4.9 TB/s, 56 us of them (6 of
 // these the launch's) the x columns, whose anchors cost a 128-byte line per row end and field. With
 // the division by a shared reciprocal and each such line written by neighbouring lanes at once:
-// 192^3 95 -> 91 us, 128^3 42.4 -> 40.7, the 64 uneven blocks (four launches) 206 -> 199.
+// 192^3 95 -> 92 us, 128^3 42.4 -> 41.5, the 64 uneven blocks (four launches) 206 -> 200.
 template <int G>
 __device__ void fill_ghost_cell(const BlockDesc& b, gdouble* u, long t_, int mode, int faces, int g) {
 #pragma clang fp contract(off)

@@ -122,7 +122,10 @@ int gr_level_create(gr_engine* eng, int nblocks, const gr_geom* geoms, gr_level*
 int gr_level_destroy(gr_level* lvl);
 int gr_level_upload(gr_level* lvl, int block, const double* host_u);
 int gr_level_download(gr_level* lvl, int block, double* host_u);
-/* Device address of block `block`'s state (22*stride doubles) for device-resident callers. */
+/* Device address of block `block`'s state (22*stride doubles) for device-resident callers. It is
+ * aligned to 16 bytes and need not be the start of an allocation: where rows are a multiple of 8
+ * doubles and ng is even, it lies behind the start by as much (32 bytes with 4 ghosts) as lets
+ * interior rows start on 64 bytes. A handle of the allocation (hipIpcGetMemHandle) opens at its start. */
 int gr_level_state(gr_level* lvl, int block, double** d_u);
 
 /* Brill-Lindquist data on every cell of every block, ghosts included
