@@ -619,7 +619,7 @@ void tune_put(int kind, int cls, int prec, int v) {
     g_tune[std::make_tuple(kind, cls, prec)] = v;
 }
 
-// First line of a saved table. Tables of earlier builds name stagings of the stage kernel that are gone:
+// First line of a saved table. Tables of earlier versions name stagings of the stage kernel that are gone:
 // their values 1 and 2 would now force a part shape, so their stage entries are not taken and those
 // classes keep the default.
 constexpr const char* kTuneHeader = "# granite-ccz4 tuning table, stage forms by part shape: kind class precision value";

@@ -1,5 +1,5 @@
-"""A tuning table written by an earlier build names stagings of the stage kernel that no longer exist: its
-stage entries are checked but not taken, all others are. Host-only."""
+"""A tuning table written by an earlier version of the library names stagings of the stage kernel that no
+longer exist: its stage entries are checked but not taken, all others are. Host-only."""
 import os
 
 import pytest
@@ -26,11 +26,11 @@ def test_stage_entries_of_an_old_table_are_not_taken(tmp_path):
     ga.tune_clear()
 
 
-def test_a_table_of_this_build_is_taken_whole(tmp_path):
+def test_a_current_table_is_taken_whole(tmp_path):
     _lib()
     ga.tune_clear()
     path, out = os.path.join(str(tmp_path), "new.txt"), os.path.join(str(tmp_path), "out.txt")
-    with open(path, "w") as f:  # no header: entries by hand, in this build's numbers
+    with open(path, "w") as f:  # no header: entries by hand, in the current numbers
         f.write("0 0 0 1\n0 3 0 2\n1 2 0 11\n")
     ga.tune_load(path)
     want = rows(out)
